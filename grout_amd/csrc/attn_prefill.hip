@@ -137,6 +137,15 @@ __device__ __forceinline__ void lds_dma16(const void* gbase, uint32_t voff, uint
         : "memory");
 }
 
+// A wave-uniform pointer held in SGPRs, where the compiler does not see that it
+// is uniform.
+__device__ __forceinline__ const uint16_t* uniform_ptr(const uint16_t* p) {
+    const uint64_t v = reinterpret_cast<uint64_t>(p);
+    const uint32_t lo = __builtin_amdgcn_readfirstlane(static_cast<uint32_t>(v));
+    const uint32_t hi = __builtin_amdgcn_readfirstlane(static_cast<uint32_t>(v >> 32));
+    return reinterpret_cast<const uint16_t*>(static_cast<uint64_t>(hi) << 32 | lo);
+}
+
 // f16(f32(o / l)) for f32 o and l > 0, with rl = 1/l rounded to f64: the f64
 // product o*rl is within 2^-52 (relative) of o/l, while a quotient of two f32
 // values in the f32 normal range is never an f32 rounding midpoint and lies
@@ -163,6 +172,98 @@ __device__ __forceinline__ void pf_barrier() {
     asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
 }
 
+// GEMM phase of one tile: O^T += V^T P^T of the previous tile (MFMA slots 0-15:
+// key step i/4, dim block i%4; `vb`: this lane's base in its V stage), then
+// S^T = K Q^T of this tile (slots 16-31: dim step (i-16)/2, key block i%2;
+// `kb`: this lane's base in its K stage).  One software pipeline over the 32
+// slots: each slot's LDS operand is read kPfAhead slots before its MFMA into a
+// ring of registers, so LDS latency hides behind ~kPfAhead MFMAs; a
+// scheduling fence per slot keeps that order.
+__device__ __forceinline__ void pf_gemm(const unsigned char* kb, const unsigned char* vb, const half8_t (&qop)[8],
+                                        const half8_t (&pop)[4], float16_t (&o)[4], float16_t (&s)[2]) {
+    constexpr int kRing = kPfAhead + 1;
+    auto read_op = [&](int i) {
+        if (i < 16) {
+            // V^T[32 dims of block i%4, 16 keys of step i/4].
+            const unsigned char* p0 = vb + 256 * (i >> 2) + 64 * (i & 3);
+            return cat(lds_read_tr16(reinterpret_cast<const half_t*>(p0)),
+                       lds_read_tr16(reinterpret_cast<const half_t*>(p0 + 8 * kPfVBlock)));
+        }
+        // K[32 keys of block i%2, 16 dims of step (i-16)/2].
+        return *reinterpret_cast<const half8_t*>(kb + 512 * (i & 1) + 32 * ((i - 16) >> 1));
+    };
+#pragma unroll
+    for (int mb = 0; mb < 2; ++mb)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) s[mb][r] = 0.0f;
+    half8_t ring[kRing];
+    // Issue priority above the softmax-phase wave on the same SIMD while
+    // feeding the matrix core (measured: ~1% faster; raising the softmax
+    // phase instead does nothing).
+    __builtin_amdgcn_s_setprio(2);
+#pragma unroll
+    for (int i = 0; i < kPfAhead; ++i) ring[i % kRing] = read_op(i);
+#pragma unroll
+    for (int i = 0; i < 32; ++i) {
+        if (i + kPfAhead < 32) ring[(i + kPfAhead) % kRing] = read_op(i + kPfAhead);
+        if (i < 16) {
+            o[i & 3] = mfma32x32x16(ring[i % kRing], pop[i >> 2], o[i & 3]);
+        } else {
+            s[i & 1] = mfma32x32x16(ring[i % kRing], qop[(i - 16) >> 1], s[i & 1]);
+        }
+        __builtin_amdgcn_sched_barrier(0);
+    }
+    __builtin_amdgcn_s_setprio(0);
+}
+
+// Softmax of one (already masked) tile: P = 2^(c*s - m) into `pop`, its row
+// sum into l, with the running max m raised only when it has to be.
+__device__ __forceinline__ void pf_softmax(const float16_t (&s)[2], half8_t (&pop)[4], float16_t (&o)[4],
+                                           float& m_run, float& l_run, float c) {
+    // The row sum runs in four independent f32 chains.
+    auto exp_tile = [&](float m_use) {
+        // Each chain starts from its first pair rather than from 0.0f: the
+        // compiler keeps a float 0 + x (it is not x for x = -0), and those
+        // four adds measured ~1% of the kernel's time.  p >= 0, so the
+        // sums are the same values.
+        float ps[4];
+#pragma unroll
+        for (int mb = 0; mb < 2; ++mb)
+#pragma unroll
+            for (int r = 0; r < 16; r += 2) {
+                const float p0 = __builtin_amdgcn_exp2f(fmaf(s[mb][r], c, -m_use));
+                const float p1 = __builtin_amdgcn_exp2f(fmaf(s[mb][r + 1], c, -m_use));
+                const int k = (r >> 1) & 3;
+                ps[k] = (mb == 0 && r < 8) ? (p0 + p1) : ps[k] + (p0 + p1);
+                pop[2 * mb + (r >> 3)][r & 7] = static_cast<half_t>(p0);
+                pop[2 * mb + (r >> 3)][(r & 7) + 1] = static_cast<half_t>(p1);
+            }
+        return (ps[0] + ps[1]) + (ps[2] + ps[3]);
+    };
+    float psum = exp_tile(m_run);
+    // The max is only raised when P would leave f16 range: a lane's partial
+    // row sum below 2^15 bounds each of its p below 2^15 (the test also
+    // catches inf).  Then the tile's row max becomes the running max, O and
+    // l are rescaled and P is recomputed.  Until then p <= 2^15 keeps full
+    // f16 relative precision, so the normalised result is the same function.
+    if (__any(!(psum < kPfPsumLimit))) {
+        float mx = kPfNegBig;
+#pragma unroll
+        for (int mb = 0; mb < 2; ++mb)
+#pragma unroll
+            for (int r = 0; r < 16; ++r) mx = fmaxf(mx, s[mb][r]);
+        mx = fmaxf(mx, swap_halves(mx));
+        const float m_new = fmaxf(m_run, mx * c);
+        const float alpha = __builtin_amdgcn_exp2f(m_run - m_new);
+        l_run *= alpha;
+#pragma unroll
+        for (int db = 0; db < 4; ++db) o[db] *= alpha;
+        m_run = m_new;
+        psum = exp_tile(m_run);
+    }
+    l_run += psum;
+}
+
 // Workgroup: 8 wavefronts x 32 query rows, all on query heads of one KV head.
 // Waves 0-3 (group A, one per SIMD) and 4-7 (group B) run the same per-tile
 // program one phase apart ("ping-pong"): a tile is two phases, GEMM (PV of the
@@ -182,13 +283,17 @@ constexpr int kPfRows = 32;
 // kDyn: persistent workgroups that claim tasks from the per-XCD queues above
 // instead of taking one task from blockIdx; each task runs exactly as in the
 // static grid, so the output is bit-identical.
-// kWaves = 4: group A alone (one wavefront per SIMD, no ping-pong partner), for
-// grids too small to fill the GPU: a tile step then takes one GEMM phase and
-// one softmax phase of one wavefront instead of two of each, which shortens
-// the latency of the heaviest workgroup.  Every wavefront computes exactly what
-// it computes in the 8-wavefront workgroup, so the output is bit-identical.
+// kWaves = 4: group A alone (one computing wavefront per SIMD, no ping-pong
+// partner) on 4 row tiles, and four wavefronts that only copy, for grids too
+// small to fill the GPU: twice the workgroups, and a tile step takes one GEMM
+// phase and one softmax phase.  A 1 KB copy holds up the wavefront that issues
+// it for ~100 cycles; left to the computing wavefronts, their eight copies a
+// step were ~800 of ~2850 cycles, with the copy wavefronts a step takes ~2300
+// (Qwen3-4B, 1000 tokens 24.3 -> 21.3 us; 509 tokens behind 6003 117 -> 95 us).
+// Every wavefront computes exactly what it computes in the 8-wavefront
+// workgroup, so the output is bit-identical.
 template <bool kSplit, bool kDyn, int kWaves = kPfWaves>
-__global__ __launch_bounds__(kWaves * kWave, 1) void attn_prefill_kernel(PrefillArgs a) {
+__global__ __launch_bounds__(kPfWaves * kWave, 1) void attn_prefill_kernel(PrefillArgs a) {
     static_assert(!(kSplit && kDyn), "the split-K form keeps the static grid");
     static_assert(kWaves == kPfWaves || (kWaves == 4 && !kSplit && !kDyn),
                   "the 4-wavefront form is the plain static grid only");
@@ -196,7 +301,9 @@ __global__ __launch_bounds__(kWaves * kWave, 1) void attn_prefill_kernel(Prefill
     __shared__ __attribute__((aligned(1024))) unsigned char pf_lds[kPfStages * kPfStageBytes];
 
     const int tid = threadIdx.x;
-    const int wave = __builtin_amdgcn_readfirstlane(tid / kWave);
+    const int wave_id = __builtin_amdgcn_readfirstlane(tid / kWave);
+    const bool copies_only = kWaves == 4 && wave_id >= 4;
+    const int wave = kWaves == 4 ? wave_id & 3 : wave_id;  // copy wavefront w fills blocks as wave w
     const int grp = wave >> 2;  // 0: group A, 1: group B (one phase behind)
     const int lane = tid % kWave;
     const int l32 = lane & 31;
@@ -396,8 +503,8 @@ __global__ __launch_bounds__(kWaves * kWave, 1) void attn_prefill_kernel(Prefill
                 row_base = static_cast<int64_t>(n0) * kHeadDim;
                 off = static_cast<uint32_t>(row - n0) * 256u + 16u * (ln & 15);
             }
-            lds_dma16(kh + row_base, off, kb + kPfKBlock * blk);
-            lds_dma16(vh + row_base, off, vb + kPfVBlock * blk);
+            lds_dma16(uniform_ptr(kh + row_base), off, __builtin_amdgcn_readfirstlane(kb + kPfKBlock * blk));
+            lds_dma16(uniform_ptr(vh + row_base), off, __builtin_amdgcn_readfirstlane(vb + kPfVBlock * blk));
         }
     };
 
@@ -405,8 +512,31 @@ __global__ __launch_bounds__(kWaves * kWave, 1) void attn_prefill_kernel(Prefill
     // (after the barrier that opens it), into the stage of tile t-2, whose
     // last reader (group B's PV of tile t-2, in its GEMM(t-1)) ended before
     // that barrier.
-    if (ntiles > 0) issue_tile(0, 0, std::integral_constant<bool, kDyn>{});
-    if (ntiles > 1) issue_tile(1, 1, std::integral_constant<bool, kDyn>{});
+    if (kWaves != 4 || copies_only) {
+        if (ntiles > 0) issue_tile(0, 0, std::integral_constant<bool, kDyn>{});
+        if (ntiles > 1) issue_tile(1, 1, std::integral_constant<bool, kDyn>{});
+    }
+    // Tile t is in LDS once at most the copies of tile t+1 are outstanding
+    // (vector-memory loads retire in order).
+    static_assert(kPfStages == 4, "the wait below assumes one tile in flight behind tile t");
+    auto wait_tile = [&](int t) {
+        if (t >= ntiles) return;
+        if (t + 1 < ntiles) {
+            __builtin_amdgcn_s_waitcnt(waitcnt_vm(2 * kDmaPerWave));
+        } else {
+            __builtin_amdgcn_s_waitcnt(waitcnt_vm(0));
+        }
+    };
+    if constexpr (kWaves == 4) {
+        if (copies_only) {
+            for (int t = 0; t <= ntiles; ++t) {
+                wait_tile(t);
+                pf_barrier();
+                if (t + 2 < ntiles) issue_tile(t + 2, (t + 2) % kPfStages, std::false_type{});
+            }
+            return;
+        }
+    }
 
     // Q^T (B operand): qop[kk] = Q[row0 + l32][16kk + 8hl + 0..7].
     half8_t qop[8];
@@ -456,12 +586,7 @@ __global__ __launch_bounds__(kWaves * kWave, 1) void attn_prefill_kernel(Prefill
     const uint32_t k_lane = (l32 & 15) * kPfKBlock + (l32 >> 4) * 256 + 16 * hl;
     const uint32_t v_lane = (4 * (gi >> 1) + (ii >> 2)) * kPfVBlock + 32 * (gi & 1) + 8 * (ii & 3);
 
-    // GEMM phase of tile j: O^T += V^T P^T of tile j-1 (MFMA slots 0-15:
-    // key step i/4, dim block i%4), then S^T = K Q^T of tile j (slots 16-31:
-    // dim step (i-16)/2, key block i%2).  One software pipeline over the 32
-    // slots: each slot's LDS operand is read kPfAhead slots before its MFMA
-    // into a ring of registers, so LDS latency hides behind ~kPfAhead MFMAs;
-    // a scheduling fence per slot keeps that order.
+    // GEMM phase of tile j: PV of tile j-1, then S of tile j.
     //
     // Every GEMM phase runs all 32 slots (one code path keeps register
     // allocation tight): at j = 0 the PV half multiplies P = 0 with the V
@@ -473,41 +598,8 @@ __global__ __launch_bounds__(kWaves * kWave, 1) void attn_prefill_kernel(Prefill
     // never softmaxed.  One skip condition keeps the accumulators in place.
     auto gemm_phase = [&](int j) {
         if (j > wave_tiles) return;
-        constexpr int kRing = kPfAhead + 1;
-        const unsigned char* vb = pf_lds + ((j + kPfStages - 1) % kPfStages) * kPfStageBytes + kPfKBytes + v_lane;
-        const unsigned char* kb = pf_lds + (j % kPfStages) * kPfStageBytes + k_lane;
-        auto read_op = [&](int i) {
-            if (i < 16) {
-                // V^T[32 dims of block i%4, 16 keys of step i/4].
-                const unsigned char* p0 = vb + 256 * (i >> 2) + 64 * (i & 3);
-                return cat(lds_read_tr16(reinterpret_cast<const half_t*>(p0)),
-                           lds_read_tr16(reinterpret_cast<const half_t*>(p0 + 8 * kPfVBlock)));
-            }
-            // K[32 keys of block i%2, 16 dims of step (i-16)/2].
-            return *reinterpret_cast<const half8_t*>(kb + 512 * (i & 1) + 32 * ((i - 16) >> 1));
-        };
-#pragma unroll
-        for (int mb = 0; mb < 2; ++mb)
-#pragma unroll
-            for (int r = 0; r < 16; ++r) s[mb][r] = 0.0f;
-        half8_t ring[kRing];
-        // Issue priority above the softmax-phase wave on the same SIMD while
-        // feeding the matrix core (measured: ~1% faster; raising the softmax
-        // phase instead does nothing).
-        __builtin_amdgcn_s_setprio(2);
-#pragma unroll
-        for (int i = 0; i < kPfAhead; ++i) ring[i % kRing] = read_op(i);
-#pragma unroll
-        for (int i = 0; i < 32; ++i) {
-            if (i + kPfAhead < 32) ring[(i + kPfAhead) % kRing] = read_op(i + kPfAhead);
-            if (i < 16) {
-                o[i & 3] = mfma32x32x16(ring[i % kRing], pop[i >> 2], o[i & 3]);
-            } else {
-                s[i & 1] = mfma32x32x16(ring[i % kRing], qop[(i - 16) >> 1], s[i & 1]);
-            }
-            __builtin_amdgcn_sched_barrier(0);
-        }
-        __builtin_amdgcn_s_setprio(0);
+        pf_gemm(pf_lds + (j % kPfStages) * kPfStageBytes + k_lane,
+                pf_lds + ((j + kPfStages - 1) % kPfStages) * kPfStageBytes + kPfKBytes + v_lane, qop, pop, o, s);
     };
 
     // Softmax phase of tile j: mask, running max (lazy), P = 2^(c*s - m), row sum.
@@ -536,49 +628,7 @@ __global__ __launch_bounds__(kWaves * kWave, 1) void attn_prefill_kernel(Prefill
                     if (static_cast<uint32_t>(rel) >= span) s[mb][r] = kMasked;
                 }
         }
-        // P = 2^(c*s - m) with the running max m as it stands; the row sum
-        // runs in four independent f32 chains.
-        auto exp_tile = [&](float m_use) {
-            // Each chain starts from its first pair rather than from 0.0f: the
-            // compiler keeps a float 0 + x (it is not x for x = -0), and those
-            // four adds measured ~1% of the kernel's time.  p >= 0, so the
-            // sums are the same values.
-            float ps[4];
-#pragma unroll
-            for (int mb = 0; mb < 2; ++mb)
-#pragma unroll
-                for (int r = 0; r < 16; r += 2) {
-                    const float p0 = __builtin_amdgcn_exp2f(fmaf(s[mb][r], c, -m_use));
-                    const float p1 = __builtin_amdgcn_exp2f(fmaf(s[mb][r + 1], c, -m_use));
-                    const int k = (r >> 1) & 3;
-                    ps[k] = (mb == 0 && r < 8) ? (p0 + p1) : ps[k] + (p0 + p1);
-                    pop[2 * mb + (r >> 3)][r & 7] = static_cast<half_t>(p0);
-                    pop[2 * mb + (r >> 3)][(r & 7) + 1] = static_cast<half_t>(p1);
-                }
-            return (ps[0] + ps[1]) + (ps[2] + ps[3]);
-        };
-        float psum = exp_tile(m_run);
-        // The max is only raised when P would leave f16 range: a lane's partial
-        // row sum below 2^15 bounds each of its p below 2^15 (the test also
-        // catches inf).  Then the tile's row max becomes the running max, O and
-        // l are rescaled and P is recomputed.  Until then p <= 2^15 keeps full
-        // f16 relative precision, so the normalised result is the same function.
-        if (__any(!(psum < kPfPsumLimit))) {
-            float mx = kPfNegBig;
-#pragma unroll
-            for (int mb = 0; mb < 2; ++mb)
-#pragma unroll
-                for (int r = 0; r < 16; ++r) mx = fmaxf(mx, s[mb][r]);
-            mx = fmaxf(mx, swap_halves(mx));
-            const float m_new = fmaxf(m_run, mx * c);
-            const float alpha = __builtin_amdgcn_exp2f(m_run - m_new);
-            l_run *= alpha;
-#pragma unroll
-            for (int db = 0; db < 4; ++db) o[db] *= alpha;
-            m_run = m_new;
-            psum = exp_tile(m_run);
-        }
-        l_run += psum;
+        pf_softmax(s, pop, o, m_run, l_run, c);
     };
 
     // Tile step t: group A runs GEMM(t) then softmax(t), group B softmax(t-1)
@@ -588,17 +638,8 @@ __global__ __launch_bounds__(kWaves * kWave, 1) void attn_prefill_kernel(Prefill
     // barriers, one at the start of each step.  Tile t+2 is issued after the
     // barrier of step t into the stage of tile t-2, whose last reader (group
     // B's GEMM(t-1), the PV of tile t-2) ended before that barrier.
-    static_assert(kPfStages == 4, "the wait below assumes one tile in flight behind tile t");
     auto open_tile_step = [&](int t) {
-        if (t < ntiles) {
-            // Tile t is in LDS once at most the copies of tile t+1 are
-            // outstanding (vector-memory loads retire in order).
-            if (t + 1 < ntiles) {
-                __builtin_amdgcn_s_waitcnt(waitcnt_vm(2 * kDmaPerWave));
-            } else {
-                __builtin_amdgcn_s_waitcnt(waitcnt_vm(0));
-            }
-        }
+        if constexpr (kWaves != 4) wait_tile(t);
         pf_barrier();
     };
     // The copies of tile t+2 go out at the start of each wavefront's softmax
@@ -610,7 +651,7 @@ __global__ __launch_bounds__(kWaves * kWave, 1) void attn_prefill_kernel(Prefill
         for (int t = 0; t <= ntiles; ++t) {
             open_tile_step(t);
             gemm_phase(t);
-            if (t + 2 < ntiles) issue_tile(t + 2, (t + 2) % kPfStages, std::false_type{});
+            if (kWaves != 4 && t + 2 < ntiles) issue_tile(t + 2, (t + 2) % kPfStages, std::false_type{});
             softmax_phase(t);
         }
     } else {
@@ -931,6 +972,35 @@ static bool prefill_short_fits(const PrefillArgs& a, int cus) {
     return last_end <= static_cast<int64_t>(kSpWaves) * kPfBN && n_blocks * a.num_q_heads <= cus;
 }
 
+// Time of a grid of `blocks` workgroups (one per CU) that walk from `most` down
+// to `least` key tiles, longest first, in tile steps: one round takes the
+// longest; in a second round the k-th workgroup past the CUs follows the k-th
+// shortest of the first, and with evenly spaced lengths all those pairs have the
+// same sum.  Launch, first loads and output stores count as `fixed` steps, 3
+// more for a second workgroup on a CU.
+static int64_t prefill_rounds(int64_t blocks, int64_t cus, int64_t most, int64_t least, int64_t fixed) {
+    int64_t t = most + fixed;
+    if (blocks > cus) t = max(t, 2 * most - (most - least) * (2 * cus - 1) / (blocks - 1) + fixed + 3);
+    return t;
+}
+
+// Whether 4-tile workgroups (blocks4) beat 8-tile ones (blocks8).  A step of
+// the former takes 4/5 of a step of the latter (0.96 against 1.22 us), so they
+// lose once the grid needs as many rounds of workgroups more.  Measured, 4 against 8
+// tiles: 32/8 heads 1500 tokens 28.7 / 35.8 us, 2048 45.0 / 50.1, 3000 93.9 /
+// 82.0; 64/8 heads 1024 tokens 27.6 / 29.9, 2048 88.3 / 73.5; 16/8 heads 4096
+// tokens 79.8 / 90.8; 32/8 heads, 1024 tokens behind 8192, 157 / 168.
+static bool prefill_narrow_wins(const PrefillArgs& a, int64_t blocks8, int64_t blocks4, int64_t cus) {
+    if (blocks4 <= cus) return true;
+    if (blocks4 > 2 * cus) return false;
+    const int64_t most = (min(static_cast<int64_t>(a.kv_len),
+                              static_cast<int64_t>(a.query_start) + kPfRows * static_cast<int64_t>(a.n_pos_tiles)) +
+                          kPfBN - 1) / kPfBN;
+    const int64_t least = (min(static_cast<int64_t>(a.kv_len), static_cast<int64_t>(a.query_start) + kPfRows) +
+                           kPfBN - 1) / kPfBN;
+    return 4 * prefill_rounds(blocks4, cus, most, least, 5) <= 5 * prefill_rounds(blocks8, cus, most, least, 4);
+}
+
 static int32_t launch_prefill(PrefillArgs a, int num_kv_heads, hipStream_t stream) {
     a.n_pos_tiles = (a.q_len + kPfRows - 1) / kPfRows;
     a.tasks_per_head = a.n_pos_tiles * a.group;
@@ -947,12 +1017,11 @@ static int32_t launch_prefill(PrefillArgs a, int num_kv_heads, hipStream_t strea
                            dim3(kSpWaves * kWave), 0, stream, a);
         return launch_status();
     }
-    if (2 * blocks <= static_cast<int64_t>(cus)) {
-        // At most half the CUs busy: 4-wavefront workgroups, twice as many.
-        a.blocks_per_head = (a.tasks_per_head + 3) / 4;
-        const int64_t blocks4 = static_cast<int64_t>(a.blocks_per_head) * num_kv_heads;
-        hipLaunchKernelGGL((attn_prefill_kernel<false, false, 4>), dim3(static_cast<unsigned>(blocks4)),
-                           dim3(4 * kWave), 0, stream, a);
+    const int64_t bph4 = (static_cast<int64_t>(a.tasks_per_head) + 3) / 4;
+    if (prefill_narrow_wins(a, blocks, bph4 * num_kv_heads, cus)) {
+        a.blocks_per_head = static_cast<int>(bph4);
+        hipLaunchKernelGGL((attn_prefill_kernel<false, false, 4>), dim3(static_cast<unsigned>(bph4 * num_kv_heads)),
+                           dim3(kPfWaves * kWave), 0, stream, a);
         return launch_status();
     }
     hipLaunchKernelGGL((attn_prefill_kernel<false, false>), dim3(static_cast<unsigned>(blocks)),

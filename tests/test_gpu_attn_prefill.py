@@ -142,6 +142,39 @@ def test_small_grid_workgroup_shape_is_bit_identical(gpu, S, G, qs):
     assert_close_attn(small[::37], ref[::37], "4-wavefront workgroups, sampled rows")
 
 
+@pytest.mark.parametrize("S,G,hkv,qs", [
+    (1000, 4, 8, 0),    # one round of 4-tile workgroups, ragged last tile
+    (1024, 8, 8, 0),    # two rounds: 512 workgroups on 256 CUs
+    (33, 3, 2, 700),    # a handful of workgroups, tasks past the end, 12 tiles
+    (65, 1, 5, 0),      # shortest walks: 1 and 2 tiles
+])
+def test_narrow_workgroups_are_bit_identical(gpu, S, G, hkv, qs):
+    """4-tile workgroups (computing and copying wavefronts apart) against the
+    8-tile grid, which the same problem takes once more KV heads fill the GPU
+    several times over: the shared heads agree bit for bit."""
+    import torch
+
+    cus = torch.cuda.get_device_properties(0).multi_processor_count
+    n_pos = -(-S // 32)
+    hkv_big = hkv * (-(-4 * cus // (-(-n_pos * G // 8) * hkv)))
+    print(f"[prefill narrow] S={S} G={G} Hkv {hkv} vs {hkv_big}", flush=True)
+    # Past the short form's 8 key tiles, or past its one workgroup per CU.
+    kv_pad = 520 if qs + S <= 512 else 0
+    g = torch.Generator(device="cuda").manual_seed(500 + S)
+    q, kc, vc = (torch.randn(s, generator=g, device="cuda", dtype=torch.float16)
+                 for s in ((S, hkv_big * G, D), (hkv_big, qs + S + kv_pad, D), (hkv_big, qs + S + kv_pad, D)))
+    import grout_amd
+
+    kv_len = qs + S + kv_pad
+    small = torch.full((S, hkv * G, D), float("nan"), dtype=torch.float16, device="cuda")
+    grout_amd.attend_prefill(q[:, :hkv * G].contiguous(), kc[:hkv].contiguous(), vc[:hkv].contiguous(),
+                             small, qs + kv_pad, kv_len=kv_len)
+    big = torch.empty_like(q)
+    grout_amd.attend_prefill(q, kc, vc, big, qs + kv_pad, kv_len=kv_len)
+    torch.cuda.synchronize()
+    assert torch.equal(small.view(torch.int16), big[:, :hkv * G].contiguous().view(torch.int16))
+
+
 def _short_form_applies(cus, hq, S, qs, kv_len):
     """The host rule of the short form: every 32-row block needs at most 8 key
     tiles of 64, and one workgroup per (query head, row block) fits the CUs."""
