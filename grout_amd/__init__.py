@@ -207,7 +207,9 @@ def attend_prefill(q, k_cache, v_cache, out, position_start: int,
     kv_len defaults to position_start + q_len (:5638); qk_scale to 1/sqrt(D) in
     f32 (:5601).  With `sched_counters` (prefill_sched_counters()) the launch
     uses the dynamic per-XCD schedule (grout_attn_prefill_sched); the result
-    is bit-identical to the static grid's."""
+    is bit-identical to the static grid's.  A few rows behind many keys take
+    grout_attn_prefill_ws with scratch from torch's allocator, except while the
+    current stream is being captured."""
     _ensure(q.dim() == 3, f"q must be rank 3 [seqlen, heads, head_dim], got {list(q.shape)}")
     q_len, Hq, D = q.shape
     Hkv, MS, _ = k_cache.shape
@@ -221,17 +223,42 @@ def attend_prefill(q, k_cache, v_cache, out, position_start: int,
         _f16(t, n)
     args = (_ptr(q), _ptr(k_cache), _ptr(v_cache), _ptr(out), float(qk_scale), Hq, Hkv, D, q_len,
             int(kv_len), int(position_start), MS)
-    if sched_counters is None:
-        _check(lib().grout_attn_prefill(*args, _stream()), "attn_prefill")
-    else:
+    if sched_counters is not None:
         _ensure(sched_counters.is_cuda and sched_counters.is_contiguous(),
                 "sched_counters must be a contiguous device tensor")
         _ensure(sched_counters.numel() * sched_counters.element_size()
                 >= lib().grout_attn_prefill_sched_counter_bytes(),
                 "sched_counters is smaller than grout_attn_prefill_sched_counter_bytes()")
+    workspace = None
+    if kv_len > 512:  # shorter key ranges never split
+        workspace = _prefill_workspace(q.device, Hq, Hkv, D, q_len, int(kv_len), int(position_start), MS)
+    if workspace is not None:
+        _check(lib().grout_attn_prefill_ws(
+            *args, None if sched_counters is None else _ptr(sched_counters), _ptr(workspace),
+            workspace.numel(), _stream()), "attn_prefill_ws")
+    elif sched_counters is None:
+        _check(lib().grout_attn_prefill(*args, _stream()), "attn_prefill")
+    else:
         _check(lib().grout_attn_prefill_sched(*args, _ptr(sched_counters), _stream()),
                "attn_prefill_sched")
     return out
+
+
+def _prefill_workspace(device, *sizes):
+    """Scratch of grout_attn_prefill_ws for these sizes from torch's allocator,
+    on the current stream; None where the call runs without: its keys are not
+    split, the stream is capturing (a graph would keep writing memory that the
+    allocator has handed on), or there is no memory left."""
+    nbytes = lib().grout_attn_prefill_workspace_bytes(*sizes)
+    if nbytes <= 0:
+        return None
+    torch = _torch()
+    if torch.cuda.is_current_stream_capturing():
+        return None
+    try:
+        return torch.empty((nbytes,), dtype=torch.uint8, device=device)
+    except torch.cuda.OutOfMemoryError:
+        return None
 
 
 def prefill_sched_counters(device="cuda"):

@@ -80,6 +80,9 @@ SIGNATURES = {
     "grout_attn_prefill": (c_i32, [c_vp] * 4 + [c_f32] + [c_i32] * 7 + [c_vp]),
     "grout_attn_prefill_sched": (c_i32, [c_vp] * 4 + [c_f32] + [c_i32] * 7 + [c_vp, c_vp]),
     "grout_attn_prefill_sched_counter_bytes": (c_i64, []),
+    "grout_attn_prefill_ws": (
+        c_i32, [c_vp] * 4 + [c_f32] + [c_i32] * 7 + [c_vp, c_vp, c_i64, c_vp]),
+    "grout_attn_prefill_workspace_bytes": (c_i64, [c_i32] * 7),
     "grout_attn_prefill_split": (c_i32, [c_vp] * 5 + [c_f32] + [c_i32] * 11 + [c_vp]),
     "grout_attn_prefill_split_merge": (c_i32, [c_vp] * 3 + [c_i32] * 6 + [c_vp]),
     "grout_attn_prefill_split_partial_bytes": (c_i64, [c_i32] * 6),

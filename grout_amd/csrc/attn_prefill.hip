@@ -216,10 +216,48 @@ __device__ __forceinline__ void pf_gemm(const unsigned char* kb, const unsigned 
     __builtin_amdgcn_s_setprio(0);
 }
 
+// The GEMM phase of half a tile (32 keys: V rows of key steps 0-1 at `vb`, K
+// rows of one key block at `kb`): 8 PV and 8 S MFMAs, alternating, because the
+// 8 S MFMAs of one key block are one accumulation chain.
+__device__ __forceinline__ void pf_gemm_half(const unsigned char* kb, const unsigned char* vb,
+                                             const half8_t (&qop)[8], const half8_t (&pop)[2],
+                                             float16_t (&o)[4], float16_t (&s)[1]) {
+    constexpr int kRing = kPfAhead + 1;
+    auto read_op = [&](int i) {
+        const int n = i >> 1;
+        if ((i & 1) == 0) {
+            const unsigned char* p0 = vb + 256 * (n >> 2) + 64 * (n & 3);
+            return cat(lds_read_tr16(reinterpret_cast<const half_t*>(p0)),
+                       lds_read_tr16(reinterpret_cast<const half_t*>(p0 + 8 * kPfVBlock)));
+        }
+        return *reinterpret_cast<const half8_t*>(kb + 32 * n);
+    };
+#pragma unroll
+    for (int r = 0; r < 16; ++r) s[0][r] = 0.0f;
+    half8_t ring[kRing];
+    __builtin_amdgcn_s_setprio(2);
+#pragma unroll
+    for (int i = 0; i < kPfAhead; ++i) ring[i % kRing] = read_op(i);
+#pragma unroll
+    for (int i = 0; i < 16; ++i) {
+        if (i + kPfAhead < 16) ring[(i + kPfAhead) % kRing] = read_op(i + kPfAhead);
+        const int n = i >> 1;
+        if ((i & 1) == 0) {
+            o[n & 3] = mfma32x32x16(ring[i % kRing], pop[n >> 2], o[n & 3]);
+        } else {
+            s[0] = mfma32x32x16(ring[i % kRing], qop[n], s[0]);
+        }
+        __builtin_amdgcn_sched_barrier(0);
+    }
+    __builtin_amdgcn_s_setprio(0);
+}
+
 // Softmax of one (already masked) tile: P = 2^(c*s - m) into `pop`, its row
 // sum into l, with the running max m raised only when it has to be.
-__device__ __forceinline__ void pf_softmax(const float16_t (&s)[2], half8_t (&pop)[4], float16_t (&o)[4],
-                                           float& m_run, float& l_run, float c) {
+// kBlocks: 32-key blocks of the tile (2: the grid's 64 keys, 1: half a tile).
+template <int kBlocks>
+__device__ __forceinline__ void pf_softmax(const float16_t (&s)[kBlocks], half8_t (&pop)[2 * kBlocks],
+                                           float16_t (&o)[4], float& m_run, float& l_run, float c) {
     // The row sum runs in four independent f32 chains.
     auto exp_tile = [&](float m_use) {
         // Each chain starts from its first pair rather than from 0.0f: the
@@ -228,7 +266,7 @@ __device__ __forceinline__ void pf_softmax(const float16_t (&s)[2], half8_t (&po
         // sums are the same values.
         float ps[4];
 #pragma unroll
-        for (int mb = 0; mb < 2; ++mb)
+        for (int mb = 0; mb < kBlocks; ++mb)
 #pragma unroll
             for (int r = 0; r < 16; r += 2) {
                 const float p0 = __builtin_amdgcn_exp2f(fmaf(s[mb][r], c, -m_use));
@@ -249,7 +287,7 @@ __device__ __forceinline__ void pf_softmax(const float16_t (&s)[2], half8_t (&po
     if (__any(!(psum < kPfPsumLimit))) {
         float mx = kPfNegBig;
 #pragma unroll
-        for (int mb = 0; mb < 2; ++mb)
+        for (int mb = 0; mb < kBlocks; ++mb)
 #pragma unroll
             for (int r = 0; r < 16; ++r) mx = fmaxf(mx, s[mb][r]);
         mx = fmaxf(mx, swap_halves(mx));
@@ -628,7 +666,7 @@ __global__ __launch_bounds__(kPfWaves * kWave, 1) void attn_prefill_kernel(Prefi
                     if (static_cast<uint32_t>(rel) >= span) s[mb][r] = kMasked;
                 }
         }
-        pf_softmax(s, pop, o, m_run, l_run, c);
+        pf_softmax<2>(s, pop, o, m_run, l_run, c);
     };
 
     // Tile step t: group A runs GEMM(t) then softmax(t), group B softmax(t-1)
@@ -961,6 +999,351 @@ __global__ __launch_bounds__(kSpWaves * kWave, 1) void attn_prefill_short_kernel
         store_half8(a.out + (static_cast<int64_t>(row0 + row) * a.num_q_heads + qh) * kHeadDim + 8 * d8, h);
 }
 
+// Key-split prefill, for a few query rows behind many keys (a chunk of a prompt,
+// drafted tokens checked against a long context), where the grids above leave
+// most CUs idle and walk the keys in sequence.  gridDim.y workgroups share a
+// row block's keys and leave f32 partials (O, m, l) in a workspace, which
+// attn_prefill_split32_merge_kernel combines.
+//  * Rows are packed position-major over the query heads of the KV head: tile
+//    row i is position i / G, head i % G.  A few positions then fill a tile
+//    (7 rows of 4 heads are one tile, not four).
+//  * Workgroup = 4 row tiles; two wavefronts share a tile and take the first and
+//    the second 32 keys of every 64-key tile.  Group A (waves 0-3) and group B
+//    (waves 4-7) ping-pong as in the grid above, half a tile per phase; waves
+//    8-11 only copy.  (12 wavefronts leave 168 VGPRs each; half a tile needs
+//    154.)  At the end each wavefront takes over half of its partner's O
+//    through LDS, so a row tile leaves one partial per split.
+//  * LDS: four K and four V slots.  The copy wavefronts issue V(t+2) and K(t+3)
+//    after the barrier of step t, into the slots that GEMM(t-1) read last, three
+//    steps before GEMM(t+2) and GEMM(t+3) need them.
+// Bound by the copies with one or two row tiles per KV head (a CU takes ~40
+// bytes a cycle into LDS, HBM gives each ~28), by the phases' fixed latencies
+// (~2000 cycles a 64-key step) with more.  Measured, unsplit -> split kernel and
+// merge: 32/8 heads, 7 rows behind 12001 keys 166 -> 17.0 us (2.9 TB/s of K/V),
+// 509 behind 6003 95 -> 65; 64/8 heads, 10 behind 28683 389 -> 34 (3.5 TB/s);
+// 16/8 heads, 5 behind 3000 45 -> 10.8.
+constexpr int kPrWaves = 8;      // computing wavefronts
+constexpr int kPrCopyWaves = 4;  // and copying ones
+constexpr int kPrThreads = (kPrWaves + kPrCopyWaves) * kWave;
+constexpr int kPrTiles = 4;  // row tiles per workgroup
+constexpr int kPrSlots = 4;
+constexpr int kPrLdsBytes = kPrSlots * (kPfKBytes + kPfVBytes);
+constexpr int kPrExchBytes = 8 * kWave * 16;       // half of O of one wavefront
+constexpr int kPrMlOff = kPrWaves * kPrExchBytes;  // then m[32], l[32] per wavefront
+constexpr int kPrPartFloats = 32 * kHeadDim;       // O of one (tile, split)
+constexpr int kPrMaxSplits = 64;
+static_assert(kPrMlOff + kPrWaves * 256 <= kPrLdsBytes, "the exchange reuses the slots");
+
+struct Split32Args {
+    const uint16_t* q;
+    const uint16_t* k_cache;
+    const uint16_t* v_cache;
+    uint16_t* out;
+    float scale_log2;
+    int num_q_heads;
+    int group;
+    int rows;             // q_len * group packed rows per KV head
+    int kv_len;
+    int query_start;
+    int max_seq_len;
+    int n_tiles;          // ceil(rows / 32)
+    int blocks_per_head;  // ceil(n_tiles / kPrTiles)
+    int num_splits;       // gridDim.y
+    float* part_o;        // [Hkv, n_tiles, num_splits][32 * 128], accumulator order
+    float* part_ml;       // [Hkv, n_tiles, num_splits][m 32, l 32]
+};
+
+__global__ __launch_bounds__(kPrThreads, 1) void attn_prefill_split32_kernel(Split32Args a) {
+    __shared__ __attribute__((aligned(1024))) unsigned char pr_lds[kPrLdsBytes];
+    const int tid = threadIdx.x;
+    const int wave = __builtin_amdgcn_readfirstlane(tid / kWave);
+    const int grp = wave >> 2;  // 0: A, 1: B (2: copies)
+    const int w4 = wave & 3;
+    const int lane = tid % kWave;
+    const int l32 = lane & 31;
+    const int hl = lane >> 5;
+
+    // The order of the grids above: a head's blocks on one XCD, heaviest first.
+    const int nb = gridDim.x;
+    int T = blockIdx.x;
+    if (nb % 8 == 0) {
+        const int hkv = nb / a.blocks_per_head;
+        const int x = T % 8, i = T / 8;
+        if (hkv < 8 && 8 % hkv == 0) {
+            const int hx = 8 / hkv;
+            T = (x / hx) * a.blocks_per_head + i * hx + x % hx;
+        } else {
+            T = x * (nb / 8) + i;
+        }
+    }
+    const int kvh = T / a.blocks_per_head;
+    const int u0 = (T % a.blocks_per_head) * kPrTiles;
+    const bool task_ok = u0 + w4 < a.n_tiles;
+    const int pt = a.n_tiles - 1 - (u0 + w4);  // row tile, heaviest first
+    // Keys of row tile p end at the limit of its last position.
+    auto tile_end = [&](int p) {
+        return min(a.kv_len, a.query_start + min(32 * p + 31, a.rows - 1) / a.group + 1);
+    };
+    const int blk_kv_end = tile_end(a.n_tiles - 1 - u0);
+    // Split y's tiles: an even share of the workgroup's.
+    const int64_t n_kt = (blk_kv_end + kPfBN - 1) / kPfBN;
+    const int tile0 = static_cast<int>(n_kt * blockIdx.y / a.num_splits);
+    const int tile1 = static_cast<int>(n_kt * (blockIdx.y + 1) / a.num_splits);
+    const int steps = tile1 - tile0;
+
+    if (wave >= kPrWaves) {
+        // Copy wavefront: blocks 4 w4 + r of every tile.
+        const uint16_t* kh = a.k_cache + static_cast<int64_t>(kvh) * a.max_seq_len * kHeadDim;
+        const uint16_t* vh = a.v_cache + static_cast<int64_t>(kvh) * a.max_seq_len * kHeadDim;
+        const uint32_t lds0 = static_cast<uint32_t>(
+            (uintptr_t)((__attribute__((address_space(3))) unsigned char*)(pr_lds)));
+        auto issue = [&](int j, const uint16_t* src, uint32_t slot, int block_bytes) {
+            if (j >= steps) return;
+            const int n0 = (tile0 + j) * kPfBN;
+            const bool clamp = n0 + kPfBN > blk_kv_end;
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                const int blk = 4 * w4 + r;
+                int64_t row_base = static_cast<int64_t>(n0 + blk) * kHeadDim;
+                uint32_t off = 4096u * static_cast<uint32_t>(lane >> 4) + 16u * (lane & 15);
+                if (clamp) {
+                    // Rows at or past blk_kv_end repeat the last valid one.
+                    const int row = min(n0 + blk + 16 * (lane >> 4), blk_kv_end - 1);
+                    row_base = static_cast<int64_t>(n0) * kHeadDim;
+                    off = static_cast<uint32_t>(row - n0) * 256u + 16u * (lane & 15);
+                }
+                lds_dma16(uniform_ptr(src + row_base), off,
+                          __builtin_amdgcn_readfirstlane(slot + static_cast<uint32_t>(block_bytes * blk)));
+            }
+        };
+        auto issue_k = [&](int j) { issue(j, kh, lds0 + (j % kPrSlots) * kPfKBytes, kPfKBlock); };
+        auto issue_v = [&](int j) {
+            issue(j, vh, lds0 + kPrSlots * kPfKBytes + (j % kPrSlots) * kPfVBytes, kPfVBlock);
+        };
+        issue_k(0);
+        issue_v(0);
+        issue_k(1);
+        issue_v(1);
+        issue_k(2);
+        for (int t = 0; t <= steps; ++t) {
+            // GEMM(t) needs K(t) and V(t-1); V(t), K(t+1), V(t+1) and K(t+2),
+            // four copies each as far as they are in range, are younger.
+            if (t + 2 < steps) {
+                __builtin_amdgcn_s_waitcnt(waitcnt_vm(16));
+            } else if (t + 1 < steps) {
+                __builtin_amdgcn_s_waitcnt(waitcnt_vm(12));
+            } else if (t < steps) {
+                __builtin_amdgcn_s_waitcnt(waitcnt_vm(4));
+            } else {
+                __builtin_amdgcn_s_waitcnt(waitcnt_vm(0));
+            }
+            pf_barrier();
+            issue_v(t + 2);
+            issue_k(t + 3);
+        }
+        // The two barriers of the merge below.
+        pf_barrier();
+        pf_barrier();
+        return;
+    }
+
+    // This wavefront's tiles: tile0 + j, j < cnt.
+    int cnt = 0;
+    if (task_ok) cnt = max(0, min(tile1, (tile_end(pt) + kPfBN - 1) / kPfBN) - tile0);
+
+    // Q^T (B operand) of packed row 32 pt + l32, and that row's key limit.
+    const int ridx = min(max(32 * pt + l32, 0), a.rows - 1);
+    const int rpos = ridx / a.group;
+    const int n_end = min(a.query_start + rpos + 1, a.kv_len);
+    const bool row_ok = task_ok && 32 * pt + l32 < a.rows;
+    half8_t qop[8];
+    {
+        const uint16_t* qr = a.q + (static_cast<int64_t>(rpos) * a.num_q_heads + kvh * a.group +
+                                    (ridx - rpos * a.group)) * kHeadDim;
+#pragma unroll
+        for (int kk = 0; kk < 8; ++kk) qop[kk] = load_half8(qr + 16 * kk + 8 * hl);
+        if (!row_ok) {
+#pragma unroll
+            for (int kk = 0; kk < 8; ++kk) qop[kk] = half8_t{};
+        }
+    }
+    // Settled before the loop, as in the grid above.
+#pragma unroll
+    for (int kk = 0; kk < 8; ++kk) asm volatile("" : "+v"(qop[kk]));
+
+    float16_t o[4];
+#pragma unroll
+    for (int db = 0; db < 4; ++db)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) o[db][r] = 0.0f;
+    float m_run = kPfNegBig, l_run = 0.0f;
+    const float c = a.scale_log2;
+    float16_t s[1];
+    half8_t pop[2];
+#pragma unroll
+    for (int i = 0; i < 2; ++i) pop[i] = half8_t{};
+    // GEMM(0) multiplies P = 0 with V slot 3: zero it (finite); V(3) is copied
+    // there after the barrier of step 1.
+    {
+        uint4_t* vz = reinterpret_cast<uint4_t*>(pr_lds + kPrSlots * kPfKBytes + (kPrSlots - 1) * kPfVBytes);
+        for (int i = tid; i < kPfVBytes / 16; i += kPrWaves * kWave) vz[i] = uint4_t{0u, 0u, 0u, 0u};
+    }
+    // This wavefront's half of a tile: key block grp (K), key steps 2 grp and
+    // 2 grp + 1 (V).
+    const int gi = lane >> 4, ii = lane & 15;
+    const uint32_t k_lane = (l32 & 15) * kPfKBlock + (l32 >> 4) * 256 + 16 * hl + 512 * grp;
+    const uint32_t v_lane = kPrSlots * kPfKBytes + (4 * (gi >> 1) + (ii >> 2)) * kPfVBlock + 32 * (gi & 1) +
+                            8 * (ii & 3) + 512 * grp;
+    // First key limit in the row tile: keys below it need no mask.
+    const int n_min = min(a.query_start + max(32 * pt, 0) / a.group + 1, a.kv_len);
+
+    auto gemm_phase = [&](int j) {
+        if (j > cnt) return;
+        pf_gemm_half(pr_lds + (j % kPrSlots) * kPfKBytes + k_lane,
+                     pr_lds + ((j + kPrSlots - 1) % kPrSlots) * kPfVBytes + v_lane, qop, pop, o, s);
+    };
+    // A row may have no key in a wavefront's halves: masked scores are -inf,
+    // which leaves m = -1e30 (or the -1.3e29 of a scaled -1e30), l = 0, O = 0
+    // and so weight 0 in the merge.
+    auto softmax_phase = [&](int j) {
+        if (j < 0 || j >= cnt) return;
+        const int n0 = (tile0 + j) * kPfBN + 32 * grp;
+        if (n0 + 32 > n_min) {
+#pragma unroll
+            for (int r = 0; r < 16; ++r) {
+                const int key = n0 + 4 * hl + 8 * (r >> 2) + (r & 3);
+                if (key >= n_end) s[0][r] = -__builtin_inff();
+            }
+        }
+        pf_softmax<1>(s, pop, o, m_run, l_run, c);
+    };
+    if (grp == 0) {
+        for (int t = 0; t <= steps; ++t) {
+            pf_barrier();
+            gemm_phase(t);
+            softmax_phase(t);
+        }
+    } else {
+        for (int t = 0; t <= steps; ++t) {
+            pf_barrier();
+            softmax_phase(t - 1);
+            gemm_phase(t);
+        }
+    }
+
+    // Merge of the pair: each wavefront hands over the 64 dims the other one
+    // finishes (A keeps dim blocks 0-1, B 2-3).  No copy is outstanding: the
+    // last ones were waited for at the barrier of the last step.
+    pf_barrier();
+    const float lt = l_run + swap_halves(l_run);
+    unsigned char* exch = pr_lds + wave * kPrExchBytes;
+#pragma unroll
+    for (int k = 0; k < 8; ++k) {
+        const int i = k & 3;
+        float4_t v;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            const float lo = o[k >> 2][4 * i + e], hi = o[2 + (k >> 2)][4 * i + e];
+            v[e] = grp ? lo : hi;
+        }
+        *reinterpret_cast<float4_t*>(exch + (k * kWave + lane) * 16) = v;
+    }
+    float* ml = reinterpret_cast<float*>(pr_lds + kPrMlOff);
+    if (hl == 0) {
+        ml[wave * 64 + l32] = m_run;
+        ml[wave * 64 + 32 + l32] = lt;
+    }
+    pf_barrier();
+    if (!task_ok) return;
+    const int other = wave ^ 4;
+    const float m_o = ml[other * 64 + l32], l_o = ml[other * 64 + 32 + l32];
+    const float M = fmaxf(m_run, m_o);
+    const float f_own = __builtin_amdgcn_exp2f(m_run - M), f_o = __builtin_amdgcn_exp2f(m_o - M);
+    const float L = lt * f_own + l_o * f_o;
+    const unsigned char* oexch = pr_lds + other * kPrExchBytes;
+    float4_t x[8];
+#pragma unroll
+    for (int k = 0; k < 8; ++k) {
+        const int i = k & 3;
+        const float4_t y = *reinterpret_cast<const float4_t*>(oexch + (k * kWave + lane) * 16);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            const float own = grp ? o[2 + (k >> 2)][4 * i + e] : o[k >> 2][4 * i + e];
+            x[k][e] = own * f_own + y[e] * f_o;
+        }
+    }
+    const int64_t part = (static_cast<int64_t>(kvh) * a.n_tiles + pt) * a.num_splits + blockIdx.y;
+    float* po = a.part_o + part * kPrPartFloats + grp * (kPrPartFloats / 2);
+#pragma unroll
+    for (int k = 0; k < 8; ++k) *reinterpret_cast<float4_t*>(po + (k * kWave + lane) * 4) = x[k];
+    if (grp == 0 && hl == 0) {
+        a.part_ml[part * 64 + l32] = M;
+        a.part_ml[part * 64 + 32 + l32] = L;
+    }
+}
+
+// Merge of the key splits.  Workgroup (row tile, dim block of
+// 32): the split weights w_s = 2^(m_s - M) of the 32 rows go to LDS, then
+// thread t sums float4 t of the block over the splits (coalesced, 16 bytes a
+// thread) and the block leaves through LDS in 64-byte row pieces.
+__global__ __launch_bounds__(256) void attn_prefill_split32_merge_kernel(Split32Args a) {
+    __shared__ float s_w[kPrMaxSplits * 32];
+    __shared__ float s_red[8 * 32];
+    __shared__ float s_sum[8 * 32];
+    __shared__ __attribute__((aligned(16))) half_t s_out[32 * 40];
+    const int tid = threadIdx.x;
+    const int kvh = static_cast<int>(blockIdx.x) / a.n_tiles;
+    const int pt = static_cast<int>(blockIdx.x) % a.n_tiles;
+    const int db = blockIdx.y;
+    const int NS = a.num_splits;
+    const int64_t part = static_cast<int64_t>(blockIdx.x) * NS;
+    const float* ml = a.part_ml + part * 64;
+    const int row = tid & 31, sg = tid >> 5;
+    float mx = kPfNegBig;
+    for (int s = sg; s < NS; s += 8) mx = fmaxf(mx, ml[s * 64 + row]);
+    s_red[sg * 32 + row] = mx;
+    __syncthreads();
+#pragma unroll
+    for (int g = 0; g < 8; ++g) mx = fmaxf(mx, s_red[g * 32 + row]);
+    float sum = 0.0f;
+    for (int s = sg; s < NS; s += 8) {
+        const float w = __builtin_amdgcn_exp2f(ml[s * 64 + row] - mx);
+        s_w[s * 32 + row] = w;
+        sum += w * ml[s * 64 + 32 + row];
+    }
+    s_sum[sg * 32 + row] = sum;
+    __syncthreads();
+    // tid = i * 64 + lane: dims 32 db + 8 i + 4 hl + [0, 4) of row lane % 32.
+    const int i = tid >> 6, hl = (tid >> 5) & 1;
+    const float* po = a.part_o + part * kPrPartFloats + (db * 256 + tid) * 4;
+    float4_t acc = {0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll 8
+    for (int s = 0; s < NS; ++s) {
+        const float4_t v = *reinterpret_cast<const float4_t*>(po + static_cast<int64_t>(s) * kPrPartFloats);
+        const float w = s_w[s * 32 + row];
+#pragma unroll
+        for (int e = 0; e < 4; ++e) acc[e] += w * v[e];
+    }
+    float L = 0.0f;
+#pragma unroll
+    for (int g = 0; g < 8; ++g) L += s_sum[g * 32 + row];
+    const double rl = 1.0 / static_cast<double>(fmaxf(L, 1.0e-8f));
+    half4_t h;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) h[e] = div_to_half(acc[e], rl);
+    *reinterpret_cast<half4_t*>(s_out + row * 40 + 8 * i + 4 * hl) = h;
+    __syncthreads();
+    if (tid < 128) {
+        const int r = tid >> 2, j = tid & 3;
+        const int idx = 32 * pt + r;
+        if (idx < a.rows) {
+            const int pos = idx / a.group;
+            uint16_t* dst = a.out + (static_cast<int64_t>(pos) * a.num_q_heads + kvh * a.group + (idx - pos * a.group)) * kHeadDim;
+            store_half8(dst + 32 * db + 8 * j, *reinterpret_cast<const half8_t*>(s_out + r * 40 + 8 * j));
+        }
+    }
+}
+
 // The short form applies when every row block needs at most kSpWaves key
 // tiles and the (query head, row block) pairs number at most one per CU.
 // (The last row block's key range ends at min(kv_len, query_start + 32 *
@@ -1054,6 +1437,82 @@ static int32_t launch_prefill_sched(PrefillArgs a, int num_kv_heads, uint32_t* s
     return launch_status();
 }
 
+// How a launch is split over its keys; num_splits 0: it is not.
+struct Split32Plan {
+    int n_tiles, blocks_per_head, num_splits;
+};
+
+// Splits only where the 4-tile workgroups leave at least half the CUs idle and
+// the short form does not apply, and only when the estimate says it pays by a
+// tenth.  Estimates in ns, fitted to the measurements at the kernel and here:
+// unsplit 960 per key tile + 5000; split 870 per key tile of a split + 8000
+// (second launch, more stores) + the partials' way out and back at 3.5 TB/s.
+// 8/1 heads, 300 rows behind 1000 keys: 1 / 2 / 4 / 8 splits 23.7 / 18.3 / 15.9 /
+// 16.7 us; 32/8 heads, 7 behind 12001: 16 / 24 / 32 splits 18.3 / 17.0 / 18.1;
+// 16/8 heads, 512 behind 600: 1 / 2 splits 21.3 / 20.7; a 927-token prompt 19.0 /
+// 24.8 (paired, one split 18.5).
+static Split32Plan split32_plan(const PrefillArgs& a, int num_kv_heads, int cus) {
+    Split32Plan p = {};
+    const int64_t rows = static_cast<int64_t>(a.q_len) * a.group;
+    const int64_t n_tiles = (rows + 31) / 32;
+    const int64_t bph = (n_tiles + kPrTiles - 1) / kPrTiles;
+    const int64_t blocks = bph * num_kv_heads;
+    if (2 * blocks > cus || prefill_short_fits(a, cus)) return p;
+    const int64_t end = min(static_cast<int64_t>(a.kv_len), static_cast<int64_t>(a.query_start) + a.q_len);
+    const int64_t key_tiles = (end + kPfBN - 1) / kPfBN;
+    // The fixed cost alone exceeds what a short walk can save; callers skip the
+    // question for kv_len <= 512.
+    if (key_tiles <= 8) return p;
+    const int64_t part_bytes = n_tiles * num_kv_heads * (kPrPartFloats + 64) * 4;
+    int64_t best = (960 * key_tiles + 5000) * 9 / 10;
+    const int64_t most = min(min(static_cast<int64_t>(kPrMaxSplits), cus / blocks), key_tiles);
+    for (int64_t ns = 2; ns <= most; ++ns) {
+        const int64_t t = 870 * ((key_tiles + ns - 1) / ns) + 8000 + 2 * part_bytes * ns / 3500;
+        if (t < best) {
+            best = t;
+            p.num_splits = static_cast<int>(ns);
+        }
+    }
+    p.n_tiles = static_cast<int>(n_tiles);
+    p.blocks_per_head = static_cast<int>(bph);
+    return p;
+}
+
+static int64_t split32_workspace_bytes(const Split32Plan& p, int num_kv_heads) {
+    return static_cast<int64_t>(num_kv_heads) * p.n_tiles * p.num_splits * (kPrPartFloats + 64) * 4;
+}
+
+static int32_t launch_prefill_split32(const PrefillArgs& a, const Split32Plan& p, int num_kv_heads, void* workspace,
+                                      hipStream_t stream) {
+    Split32Args b = {};
+    b.q = a.q;
+    b.k_cache = a.k_cache;
+    b.v_cache = a.v_cache;
+    b.out = a.out;
+    b.scale_log2 = a.scale_log2;
+    b.num_q_heads = a.num_q_heads;
+    b.group = a.group;
+    b.rows = a.q_len * a.group;
+    b.kv_len = a.kv_len;
+    // A start at or past kv_len sees every key, as kv_len itself does.
+    b.query_start = min(a.query_start, a.kv_len);
+    b.max_seq_len = a.max_seq_len;
+    b.n_tiles = p.n_tiles;
+    b.blocks_per_head = p.blocks_per_head;
+    b.num_splits = p.num_splits;
+    const int64_t parts = static_cast<int64_t>(num_kv_heads) * p.n_tiles * p.num_splits;
+    b.part_o = static_cast<float*>(workspace);
+    b.part_ml = b.part_o + parts * kPrPartFloats;
+    hipLaunchKernelGGL(attn_prefill_split32_kernel,
+                       dim3(static_cast<unsigned>(p.blocks_per_head * num_kv_heads), static_cast<unsigned>(p.num_splits)),
+                       dim3(kPrThreads), 0, stream, b);
+    const int32_t st = launch_status();
+    if (st != GROUT_OK) return st;
+    hipLaunchKernelGGL(attn_prefill_split32_merge_kernel, dim3(static_cast<unsigned>(num_kv_heads * p.n_tiles), 4),
+                       dim3(256), 0, stream, b);
+    return launch_status();
+}
+
 // Merge of the split-K partials (prefill_splitk_reduce_merge,
 // src/kernels.rs:2151-2323): thread = (row < q_len, q head, 8 dims); weights
 // w_s = 2^(lse_s - max) / max(sum, 1e-8), out = f16(sum_s w_s * att_s).
@@ -1120,24 +1579,43 @@ static int64_t prefill_split_rows(int32_t num_q_heads, int32_t q_len, int32_t bl
 
 using namespace grout;
 
-// Shared by both prefill entry points: the ensure!s of
-// attend_seq_arc_into_ctx_with_position (src/model.rs:5564-5637) on sizes, then
-// the static grid (sched == nullptr) or the dynamic schedule.
-static int32_t prefill_entry(const uint16_t* q, const uint16_t* k_cache, const uint16_t* v_cache,
-                             uint16_t* out, float qk_scale, int32_t num_q_heads,
-                             int32_t num_kv_heads, int32_t head_dim, int32_t q_len, int32_t kv_len,
-                             int32_t query_start, int32_t max_seq_len, uint32_t* sched,
-                             grout_stream_t stream) {
-    GROUT_REQUIRE_PTR(q);
-    GROUT_REQUIRE_PTR(k_cache);
-    GROUT_REQUIRE_PTR(v_cache);
-    GROUT_REQUIRE_PTR(out);
+// Size checks shared by the prefill entry points: the ensure!s of
+// attend_seq_arc_into_ctx_with_position (src/model.rs:5564-5637).
+static int32_t check_prefill_sizes(int32_t num_q_heads, int32_t num_kv_heads, int32_t head_dim, int32_t q_len,
+                                   int32_t kv_len, int32_t query_start, int32_t max_seq_len) {
     GROUT_REQUIRE(head_dim == kHeadDim, GROUT_ERR_HEAD_DIM);
     GROUT_REQUIRE(num_q_heads > 0 && num_kv_heads > 0 && num_q_heads % num_kv_heads == 0,
                   GROUT_ERR_HEADS);
     GROUT_REQUIRE(max_seq_len > 0, GROUT_ERR_SEQ_RANGE);
     GROUT_REQUIRE(q_len >= 0 && query_start >= 0, GROUT_ERR_KV_LEN);
     GROUT_REQUIRE(kv_len >= 1 && kv_len <= max_seq_len, GROUT_ERR_KV_LEN);
+    return GROUT_OK;
+}
+
+// The key-split plan of a call on the current device.
+static int32_t plan_on_device(const PrefillArgs& a, int num_kv_heads, Split32Plan* p) {
+    int dev = 0, cus = 0;
+    hipError_t e = hipGetDevice(&dev);
+    if (e == hipSuccess) e = hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev);
+    if (e != hipSuccess) return static_cast<int32_t>(e);
+    *p = split32_plan(a, num_kv_heads, cus);
+    return GROUT_OK;
+}
+
+// Shared by the prefill entry points: the key split where a workspace is given
+// and it pays, else the dynamic schedule (sched != nullptr) or the static grid.
+static int32_t prefill_entry(const uint16_t* q, const uint16_t* k_cache, const uint16_t* v_cache,
+                             uint16_t* out, float qk_scale, int32_t num_q_heads,
+                             int32_t num_kv_heads, int32_t head_dim, int32_t q_len, int32_t kv_len,
+                             int32_t query_start, int32_t max_seq_len, uint32_t* sched,
+                             void* workspace, int64_t workspace_bytes, grout_stream_t stream) {
+    GROUT_REQUIRE_PTR(q);
+    GROUT_REQUIRE_PTR(k_cache);
+    GROUT_REQUIRE_PTR(v_cache);
+    GROUT_REQUIRE_PTR(out);
+    const int32_t sizes = check_prefill_sizes(num_q_heads, num_kv_heads, head_dim, q_len, kv_len, query_start,
+                                              max_seq_len);
+    if (sizes != GROUT_OK) return sizes;
     GROUT_REQUIRE(qk_scale > 0.0f && qk_scale < 1.0e30f, GROUT_ERR_ARG);
     if (q_len == 0) return GROUT_OK;
 
@@ -1154,6 +1632,13 @@ static int32_t prefill_entry(const uint16_t* q, const uint16_t* k_cache, const u
     a.kv_len = kv_len;
     a.query_start = query_start;
     a.max_seq_len = max_seq_len;
+    if (workspace != nullptr) {
+        Split32Plan p;
+        const int32_t st = plan_on_device(a, num_kv_heads, &p);
+        if (st != GROUT_OK) return st;
+        if (p.num_splits >= 2 && workspace_bytes >= split32_workspace_bytes(p, num_kv_heads))
+            return launch_prefill_split32(a, p, num_kv_heads, workspace, to_hip(stream));
+    }
     if (sched == nullptr) return launch_prefill(a, num_kv_heads, to_hip(stream));
     return launch_prefill_sched(a, num_kv_heads, sched, to_hip(stream));
 }
@@ -1164,7 +1649,7 @@ extern "C" int32_t grout_attn_prefill(const uint16_t* q, const uint16_t* k_cache
                                       int32_t q_len, int32_t kv_len, int32_t query_start,
                                       int32_t max_seq_len, grout_stream_t stream) {
     return prefill_entry(q, k_cache, v_cache, out, qk_scale, num_q_heads, num_kv_heads, head_dim,
-                         q_len, kv_len, query_start, max_seq_len, nullptr, stream);
+                         q_len, kv_len, query_start, max_seq_len, nullptr, nullptr, 0, stream);
 }
 
 extern "C" int32_t grout_attn_prefill_sched(const uint16_t* q, const uint16_t* k_cache,
@@ -1177,7 +1662,43 @@ extern "C" int32_t grout_attn_prefill_sched(const uint16_t* q, const uint16_t* k
     GROUT_REQUIRE(sched_counters != nullptr, GROUT_ERR_NULL_POINTER);
     GROUT_REQUIRE((reinterpret_cast<uintptr_t>(sched_counters) & 3u) == 0, GROUT_ERR_ALIGNMENT);
     return prefill_entry(q, k_cache, v_cache, out, qk_scale, num_q_heads, num_kv_heads, head_dim,
-                         q_len, kv_len, query_start, max_seq_len, sched_counters, stream);
+                         q_len, kv_len, query_start, max_seq_len, sched_counters, nullptr, 0, stream);
+}
+
+extern "C" int32_t grout_attn_prefill_ws(const uint16_t* q, const uint16_t* k_cache,
+                                         const uint16_t* v_cache, uint16_t* out, float qk_scale,
+                                         int32_t num_q_heads, int32_t num_kv_heads,
+                                         int32_t head_dim, int32_t q_len, int32_t kv_len,
+                                         int32_t query_start, int32_t max_seq_len,
+                                         uint32_t* sched_counters, void* workspace,
+                                         int64_t workspace_bytes, grout_stream_t stream) {
+    GROUT_REQUIRE((reinterpret_cast<uintptr_t>(sched_counters) & 3u) == 0, GROUT_ERR_ALIGNMENT);
+    GROUT_REQUIRE(aligned16(workspace), GROUT_ERR_ALIGNMENT);
+    return prefill_entry(q, k_cache, v_cache, out, qk_scale, num_q_heads, num_kv_heads, head_dim,
+                         q_len, kv_len, query_start, max_seq_len, sched_counters, workspace, workspace_bytes,
+                         stream);
+}
+
+extern "C" int64_t grout_attn_prefill_workspace_bytes(int32_t num_q_heads, int32_t num_kv_heads,
+                                                      int32_t head_dim, int32_t q_len,
+                                                      int32_t kv_len, int32_t query_start,
+                                                      int32_t max_seq_len) {
+    const int32_t sizes = check_prefill_sizes(num_q_heads, num_kv_heads, head_dim, q_len, kv_len, query_start,
+                                              max_seq_len);
+    if (sizes != GROUT_OK) return sizes;
+    if (q_len == 0) return 0;
+    PrefillArgs a = {};
+    a.num_q_heads = num_q_heads;
+    a.group = num_q_heads / num_kv_heads;
+    a.q_len = q_len;
+    a.kv_len = kv_len;
+    a.query_start = query_start;
+    a.max_seq_len = max_seq_len;
+    Split32Plan p;
+    const int32_t st = plan_on_device(a, num_kv_heads, &p);
+    // Without a device there is nothing to plan for: 0, as for a call that does not split.
+    if (st != GROUT_OK) return 0;
+    return split32_workspace_bytes(p, num_kv_heads);
 }
 
 extern "C" int64_t grout_attn_prefill_sched_counter_bytes(void) {

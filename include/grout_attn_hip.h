@@ -175,6 +175,28 @@ int32_t grout_attn_prefill_sched(const uint16_t* q, const uint16_t* k_cache,
                                  grout_stream_t stream);
 int64_t grout_attn_prefill_sched_counter_bytes(void);
 
+/* Same computation, with a device workspace for the launches whose query rows
+ * cannot fill the GPU (a chunk of a prompt, drafted tokens behind a long
+ * context): their keys are split over workgroups, f32 partials go through the
+ * workspace and a second launch merges them (within the attention tolerance of
+ * the other entry points, not bit-identical to them).  Every other launch runs
+ * as grout_attn_prefill_sched, or as grout_attn_prefill when sched_counters is
+ * NULL.
+ *   workspace: grout_attn_prefill_workspace_bytes(...) bytes for these sizes
+ *   and the current device, 16-byte aligned, contents arbitrary; NULL or fewer
+ *   bytes: no split.  Calls that overlap on one workspace race. */
+int32_t grout_attn_prefill_ws(const uint16_t* q, const uint16_t* k_cache,
+                              const uint16_t* v_cache, uint16_t* out, float qk_scale,
+                              int32_t num_q_heads, int32_t num_kv_heads, int32_t head_dim,
+                              int32_t q_len, int32_t kv_len, int32_t query_start,
+                              int32_t max_seq_len, uint32_t* sched_counters, void* workspace,
+                              int64_t workspace_bytes, grout_stream_t stream);
+/* 0 where the call would not split its keys (always for kv_len <= 512); < 0 for
+ * sizes it rejects. */
+int64_t grout_attn_prefill_workspace_bytes(int32_t num_q_heads, int32_t num_kv_heads,
+                                           int32_t head_dim, int32_t q_len, int32_t kv_len,
+                                           int32_t query_start, int32_t max_seq_len);
+
 /* -------------------------------------------------------- split-K prefill */
 /* Replaces fmha_prefill_gqa_lpt_split (src/kernels.rs:1872-2142), launched by
  * the attention microbench (benchmarks/src/bin/attention_microbench.rs:418-469)

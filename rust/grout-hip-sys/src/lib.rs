@@ -188,6 +188,18 @@ extern "C" {
         query_start: i32, max_seq_len: i32, sched_counters: *mut u32, stream: HipStream,
     ) -> i32;
     pub fn grout_attn_prefill_sched_counter_bytes() -> i64;
+    /// The same prefill with a workspace of [`grout_attn_prefill_workspace_bytes`] bytes
+    /// for launches of few query rows behind many keys; `sched_counters` may be null.
+    pub fn grout_attn_prefill_ws(
+        q: *const u16, k_cache: *const u16, v_cache: *const u16, out: *mut u16, qk_scale: f32,
+        num_q_heads: i32, num_kv_heads: i32, head_dim: i32, q_len: i32, kv_len: i32,
+        query_start: i32, max_seq_len: i32, sched_counters: *mut u32, workspace: *mut c_void,
+        workspace_bytes: i64, stream: HipStream,
+    ) -> i32;
+    pub fn grout_attn_prefill_workspace_bytes(
+        num_q_heads: i32, num_kv_heads: i32, head_dim: i32, q_len: i32, kv_len: i32,
+        query_start: i32, max_seq_len: i32,
+    ) -> i64;
     pub fn grout_attn_prefill_split(
         q: *const u16, k_cache: *const u16, v_cache: *const u16, att_partial: *mut u16,
         lse_partial: *mut f32, qk_scale: f32, num_q_heads: i32, num_kv_heads: i32, head_dim: i32,

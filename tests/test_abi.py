@@ -134,6 +134,35 @@ def test_prefill_sched_checks(L):
     assert L.grout_attn_prefill_sched_counter_bytes() == 17 * 256
 
 
+def test_prefill_ws_checks(L):
+    """grout_attn_prefill_ws: optional counters and workspace by alignment, then
+    the argument checks of grout_attn_prefill; the size query rejects the same
+    sizes."""
+    f = L.grout_attn_prefill_ws
+    ok = dict(q=A, k=A, v=A, o=A, sc=0.088, hq=4, hkv=2, D=128, ql=8, kv=8, qs=0, MS=16, c=A, w=A, n=64)
+
+    def call(**kw):
+        a = dict(ok, **kw)
+        return f(a["q"], a["k"], a["v"], a["o"], a["sc"], a["hq"], a["hkv"], a["D"], a["ql"],
+                 a["kv"], a["qs"], a["MS"], a["c"], a["w"], a["n"], S)
+
+    assert call(c=U) == -2
+    assert call(w=U) == -2
+    assert call(c=0, w=0, o=0) == -1
+    assert call(q=U) == -2
+    assert call(D=256) == -3
+    assert call(hq=5) == -4
+    assert call(kv=17) == -6
+    assert call(qs=-1) == -6
+    assert call(sc=0.0) == -9
+    assert call(ql=0) == 0
+    size = L.grout_attn_prefill_workspace_bytes
+    assert size(4, 2, 256, 8, 8, 0, 16) == -3
+    assert size(5, 2, 128, 8, 8, 0, 16) == -4
+    assert size(4, 2, 128, 8, 17, 0, 16) == -6
+    assert size(4, 2, 128, 0, 8, 0, 16) == 0
+
+
 def test_prefill_split_checks(L):
     f = L.grout_attn_prefill_split
     ok = dict(q=A, k=A, v=A, att=A, lse=A, sc=0.088, hq=8, hkv=2, D=128, ql=40, kv=40, qs=0,

@@ -165,14 +165,85 @@ def test_narrow_workgroups_are_bit_identical(gpu, S, G, hkv, qs):
                  for s in ((S, hkv_big * G, D), (hkv_big, qs + S + kv_pad, D), (hkv_big, qs + S + kv_pad, D)))
     import grout_amd
 
-    kv_len = qs + S + kv_pad
-    small = torch.full((S, hkv * G, D), float("nan"), dtype=torch.float16, device="cuda")
-    grout_amd.attend_prefill(q[:, :hkv * G].contiguous(), kc[:hkv].contiguous(), vc[:hkv].contiguous(),
-                             small, qs + kv_pad, kv_len=kv_len)
-    big = torch.empty_like(q)
-    grout_amd.attend_prefill(q, kc, vc, big, qs + kv_pad, kv_len=kv_len)
-    torch.cuda.synchronize()
-    assert torch.equal(small.view(torch.int16), big[:, :hkv * G].contiguous().view(torch.int16))
+    def run(heads):
+        out = torch.full((S, heads * G, D), float("nan"), dtype=torch.float16, device="cuda")
+        a = [t.contiguous() for t in (q[:, :heads * G], kc[:heads], vc[:heads])] + [out]
+        # The C entry point without a workspace: these shapes never split their keys.
+        status = grout_amd.lib().grout_attn_prefill(
+            *(t.data_ptr() for t in a), SCALE, heads * G, heads, D, S, qs + S + kv_pad, qs + kv_pad,
+            kc.shape[1], torch.cuda.current_stream().cuda_stream)
+        assert status == 0
+        torch.cuda.synchronize()
+        return out.view(torch.int16)
+
+    assert torch.equal(run(hkv), run(hkv_big)[:, :hkv * G])
+
+
+@pytest.mark.parametrize("hq,hkv,S,qs,kv_len,MS", [
+    (32, 8, 7, 12001, None, 12008),  # one packed tile a head, last cache row in use
+    (64, 8, 10, 5000, None, 5100),   # three tiles, the last with 16 rows
+    (6, 2, 33, 2000, None, 2100),    # G = 3: positions straddle tiles; 4 tiles, one row in the last
+    (16, 8, 1, 1000, None, 1001),    # one row, 16 key tiles
+    (5, 5, 129, 700, None, 900),     # G = 1: 5 tiles, a second workgroup with one
+    (8, 1, 300, 1000, None, 1300),   # 19 workgroups
+    (32, 8, 20, 3000, 2900, 3100),   # kv_len before the first position: no causal mask at all
+    (32, 8, 20, 3000, 3005, 3100),   # and inside the rows
+])
+def test_key_split_matches_oracle(gpu, hq, hkv, S, qs, kv_len, MS):
+    """Few rows behind many keys: keys split over workgroups, f32 partials merged
+    by a second launch; K outliers move the splits' maxima apart."""
+    import torch
+
+    import grout_amd
+
+    kv = qs + S if kv_len is None else kv_len
+    nbytes = grout_amd.lib().grout_attn_prefill_workspace_bytes(hq, hkv, D, S, kv, qs, MS)
+    tile_bytes = 32 * (D + 2) * 4 * hkv * -(-S * (hq // hkv) // 32)
+    assert nbytes >= 2 * tile_bytes and nbytes % tile_bytes == 0, "shape does not split"
+    print(f"[prefill key split] hq={hq} hkv={hkv} S={S} qs={qs} kv_len={kv} splits {nbytes // tile_bytes}", flush=True)
+    q, kc, vc = _case(600 + S, hq, hkv, S, qs, MS, scale_rows=0.01)
+    out = _run(torch, q, kc, vc, qs, kv_len=kv)
+    ref = oracle.attn_prefill_f32(q, kc, vc, SCALE, kv_len=kv, query_start=qs)
+    assert_close_attn(out, ref, f"key split hq={hq} hkv={hkv} S={S} qs={qs} kv_len={kv}")
+
+
+def test_key_split_workspace_and_capture(gpu):
+    """A workspace of NaNs or of too few bytes does not show in the output; a
+    captured call takes no scratch and replays to the unsplit result."""
+    import torch
+
+    import grout_amd
+
+    hq, hkv, S, qs = 32, 8, 5, 4000
+    q, kc, vc = (torch.from_numpy(a).cuda() for a in _case(650, hq, hkv, S, qs, qs + S))
+    L = grout_amd.lib()
+    nbytes = L.grout_attn_prefill_workspace_bytes(hq, hkv, D, S, qs + S, qs, qs + S)
+    assert nbytes > 0
+
+    def run(ws, n):
+        out = torch.full_like(q, float("nan"))
+        assert L.grout_attn_prefill_ws(
+            q.data_ptr(), kc.data_ptr(), vc.data_ptr(), out.data_ptr(), SCALE, hq, hkv, D, S, qs + S, qs,
+            qs + S, None, ws, n, torch.cuda.current_stream().cuda_stream) == 0
+        torch.cuda.synchronize()
+        return out
+
+    ws = torch.full((nbytes // 4,), float("nan"), device="cuda")
+    split = run(ws.data_ptr(), nbytes)
+    assert torch.equal(split, run(ws.data_ptr(), nbytes))
+    unsplit = run(None, 0)
+    assert torch.equal(unsplit, run(ws.data_ptr(), nbytes - 4))
+    assert_close_attn(split.cpu().numpy(), unsplit.float().cpu().numpy(), "split vs unsplit", atol=1e-3, rtol=0)
+    out = torch.empty_like(q)
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        grout_amd.attend_prefill(q, kc, vc, out, qs)
+    for _ in range(3):
+        out.fill_(float("nan"))
+        graph.replay()
+        grout_amd.attend_prefill(q, kc, vc, torch.empty_like(q), qs)
+        torch.cuda.synchronize()
+        assert torch.equal(out, unsplit)
 
 
 def _short_form_applies(cus, hq, S, qs, kv_len):
