@@ -14,12 +14,15 @@
 //  * the GEMV streams each weight row with all 256 threads of a workgroup
 //    (16-byte non-temporal loads, up to 8 rows x 3 chunks in flight per
 //    thread) and accumulates in f32 with v_dot2_f32_f16 (exact f16 products);
+//  * rows of k <= 1024 take one wavefront per two rows, and the token step's
+//    projections of rows up to 2560 normalise their input themselves;
 //  * the argmax reduces (value, index) pairs, the lowest index winning ties,
 //    in 2048-element blocks and then over the blocks.
 #include <math.h>
 
 #include "abi_util.h"
 #include "common.h"
+#include "decode_layer.h"
 
 namespace grout {
 
@@ -176,6 +179,25 @@ __device__ __forceinline__ float wave_multi_sum(float (&v)[R], int lane) {
     return v[0];
 }
 
+// Stores the R row sums of wave_multi_sum (row r in lane r * 64 / R) as outputs
+// row0 + r < m; kSilu: SiLU(row r) * row (r + R/2) as output row0 + r, r < R/2.
+template <int R, bool kSilu>
+__device__ __forceinline__ void store_wave_rows(float v, uint16_t* out, int row0, int m, int lane) {
+    constexpr int kStride = kWave / R;
+    const int o = row0 + lane / kStride;
+    if constexpr (kSilu) {
+        const float up = __shfl_xor(v, kWave / 2);
+        if (lane % kStride == 0 && lane < kWave / 2 && o < m)
+            out[o] = __builtin_bit_cast(uint16_t, silu_mul1(static_cast<half_t>(v), static_cast<half_t>(up)));
+    } else if (lane % kStride == 0 && o < m) {
+        out[o] = __builtin_bit_cast(uint16_t, static_cast<half_t>(v));
+    }
+}
+
+// Workgroup barrier that waits only for LDS traffic: global loads stay in
+// flight across it.
+__device__ __forceinline__ void lds_only_barrier() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
+
 // Workgroup b computes out rows b*R + [0, R).  kSilu (the gate_up GEMV with
 // SiLU * up in its epilogue): workgroup b computes gate rows b*R/2 + [0, R/2)
 // and the matching up rows half_m + b*R/2 + [0, R/2) as its R rows, rounds
@@ -279,6 +301,193 @@ __global__ __launch_bounds__(kGemvThreads) void gemv_f16_kernel(
         for (int w = 1; w < kGemvThreads / kWave; ++w) t += red[w][tid];
         out[row0 + tid] = __builtin_bit_cast(uint16_t, static_cast<half_t>(t));
     }
+}
+
+// Input of a GEMV with the add + RMSNorm before it folded in: x of the GEMV is
+// the RMSNorm of residual + x, and residual_out receives the sum.  A norm launch
+// of one workgroup between two GEMVs leaves HBM idle for ~5 us (2.3 us at hidden
+// 1024); folded in, every workgroup reads the rows from L2 while its weights are
+// on their way, and workgroup 0 stores the sum.
+struct NormIn {
+    const uint16_t* residual;
+    const uint16_t* x;
+    const uint16_t* weight;
+    uint16_t* residual_out;
+    float eps;
+};
+
+// Rows of at most kGemvWaveMaxK = 1024: one wavefront per R rows, no exchange
+// between wavefronts.  Lane l holds the 16-byte chunks l and l + 64 of each of
+// its rows and of x; the sums need six shuffles and no LDS.  gemv_f16_kernel
+// spreads a row over 256 threads, half of which have no chunk at k = 1024.
+// Measured, there -> here: 4096 rows 3.49 -> 3.33 us, 3072 gate/up pairs 4.47 ->
+// 4.17, 151936 rows 52 -> 47.3 us (5.9 -> 6.6 TB/s); longer rows lose (k 2048
+// 2.85 -> 3.35 us, k 2560 16.5 -> 17.6).
+// kNorm: x is the RMSNorm of in.residual + in.x (see NormIn).  Each wavefront
+// takes the row sums on c * w, c = residual + x in f32, sums c^2 beside them and
+// scales at the end: W (c * inv * w) = inv * (W (c * w)), so nothing waits for
+// inv, and the norm's output is not rounded to f16.
+constexpr int kGemvWaveMaxK = 1024;
+template <int R, bool kSilu = false, bool kNorm = false>
+__global__ __launch_bounds__(kGemvThreads) void gemv_wave_kernel(
+    const uint16_t* __restrict__ W, const uint16_t* __restrict__ x, uint16_t* __restrict__ out,
+    int m, int k, int half_m, NormIn in) {
+    static_assert(!kSilu || R >= 2, "a SiLU wavefront pairs R/2 gate rows with R/2 up rows");
+    constexpr int kOut = kSilu ? R / 2 : R;
+    constexpr int NC = kGemvWaveMaxK / 8 / kWave;
+    const int tid = threadIdx.x;
+    const int lane = tid & (kWave - 1);
+    const int wave = __builtin_amdgcn_readfirstlane(tid / kWave);
+    const int row0 = (static_cast<int>(blockIdx.x) * (kGemvThreads / kWave) + wave) * kOut;
+    if (row0 >= m) return;
+    const int nchunk = k / 8;
+    const half8_t* xc = reinterpret_cast<const half8_t*>(x);
+    half8_t wv[NC][R], xv[NC], rv[NC], nv[NC];
+#pragma unroll
+    for (int u = 0; u < NC; ++u) {
+        const int c = lane + kWave * u;
+        if (c < nchunk) {
+            if constexpr (kNorm) {
+                rv[u] = reinterpret_cast<const half8_t*>(in.residual)[c];
+                nv[u] = reinterpret_cast<const half8_t*>(in.weight)[c];
+            }
+            xv[u] = xc[c];
+#pragma unroll
+            for (int r = 0; r < R; ++r) {
+                const int o = min(row0 + r % kOut, m - 1);  // outputs past m repeat the last row
+                const int row = (kSilu && r >= kOut) ? half_m + o : o;
+                wv[u][r] = __builtin_nontemporal_load(reinterpret_cast<const half8_t*>(W + static_cast<int64_t>(row) * k) + c);
+            }
+        }
+    }
+    __builtin_amdgcn_sched_barrier(0);
+    float acc[R];
+#pragma unroll
+    for (int r = 0; r < R; ++r) acc[r] = 0.0f;
+    float ss = 0.0f;
+#pragma unroll
+    for (int u = 0; u < NC; ++u) {
+        const int c = lane + kWave * u;
+        if (c < nchunk) {
+            if constexpr (kNorm) {
+                float g[8];
+                half8_t c16;
+#pragma unroll
+                for (int e = 0; e < 8; ++e) {
+                    const float cf = static_cast<float>(rv[u][e]) + static_cast<float>(xv[u][e]);
+                    ss += cf * cf;
+                    g[e] = cf * static_cast<float>(nv[u][e]);
+                    c16[e] = static_cast<half_t>(cf);
+                }
+                if (row0 == 0) store_half8(in.residual_out + 8 * c, c16);
+#pragma unroll
+                for (int r = 0; r < R; ++r)
+#pragma unroll
+                    for (int e = 0; e < 8; ++e) acc[r] = fmaf(static_cast<float>(wv[u][r][e]), g[e], acc[r]);
+            } else {
+#pragma unroll
+                for (int r = 0; r < R; ++r) acc[r] = dot8(wv[u][r], xv[u], acc[r]);
+            }
+        }
+    }
+    float v = wave_multi_sum<R>(acc, lane);
+    if constexpr (kNorm) v *= 1.0f / sqrtf(wave_sum_f32(ss) / static_cast<float>(k) + in.eps);
+    store_wave_rows<R, kSilu>(v, out, row0, m, lane);
+}
+
+// Longer rows, up to kNormGemvMaxK = 2560, with the norm folded in (NormIn): the
+// workgroup issues the loads of the row and then of all its weights, normalises
+// the row into LDS while the weights are in flight, and each of its 8
+// wavefronts sums R rows against it (R = 2, NC = 5 chunk columns of 64 lanes).
+// The sum of squares is taken over 512 threads instead of 1024, the f16 roundings
+// are those of rms_norm_decode_kernel.  Qwen3-4B token step (36 layers, position
+// 4001) 1955 -> 1882 us; 4 wavefronts 1-2% slower, 16 wavefronts 9%.  Folding
+// the norm into gemv_f16_kernel instead (each thread normalises its own chunks)
+// 1954-2694: every 2-row workgroup then reads 15 KB of row data for 10 KB of
+// weights.  Qwen3-32B (k = 5120) keeps its norm launches: 2125 us at best against
+// 2119 for 12 layers; a row's 10 chunk columns leave too few wavefronts
+// resident to keep HBM busy through the prologue.
+constexpr int kNormGemvMaxK = 2560;
+constexpr int kNormGemvThreads = 512;
+template <int R, bool kSilu>
+__global__ __launch_bounds__(kNormGemvThreads) void norm_gemv_kernel(const uint16_t* __restrict__ W,
+                                                                     uint16_t* __restrict__ out, NormIn in, int m,
+                                                                     int k, int half_m) {
+    static_assert(!kSilu || R >= 2, "a SiLU wavefront pairs R/2 gate rows with R/2 up rows");
+    constexpr int kOut = kSilu ? R / 2 : R;
+    constexpr int NC = kNormGemvMaxK / 8 / kWave;
+    constexpr int kWaves = kNormGemvThreads / kWave;
+    static_assert(NC * kWave <= kNormGemvThreads, "one row chunk per thread");
+    __shared__ __attribute__((aligned(16))) uint16_t s_x[NC * kWave * 8];
+    __shared__ float red[kWaves];
+    const int tid = threadIdx.x;
+    const int lane = tid & (kWave - 1);
+    const int wave = __builtin_amdgcn_readfirstlane(tid / kWave);
+    const int nchunk = k / 8;
+    const int row0 = (static_cast<int>(blockIdx.x) * kWaves + wave) * kOut;
+    half8_t rv, xv, nv;
+    if (tid < nchunk) {
+        rv = load_half8(in.residual + 8 * tid);
+        xv = load_half8(in.x + 8 * tid);
+        nv = load_half8(in.weight + 8 * tid);
+    }
+    // The row's loads go out before the weights': loads return in order.
+    __builtin_amdgcn_sched_barrier(0);
+    half8_t wv[NC][R];
+#pragma unroll
+    for (int u = 0; u < NC; ++u) {
+        const int c = lane + kWave * u;
+        if (c < nchunk) {
+#pragma unroll
+            for (int r = 0; r < R; ++r) {
+                const int o = min(row0 + r % kOut, m - 1);  // outputs past m repeat the last row
+                const int row = (kSilu && r >= kOut) ? half_m + o : o;
+                wv[u][r] = __builtin_nontemporal_load(reinterpret_cast<const half8_t*>(W + static_cast<int64_t>(row) * k) + c);
+            }
+        }
+    }
+    __builtin_amdgcn_sched_barrier(0);
+    float cv[8];
+    float ss = 0.0f;
+    if (tid < nchunk) {
+#pragma unroll
+        for (int e = 0; e < 8; ++e) {
+            cv[e] = static_cast<float>(rv[e]) + static_cast<float>(xv[e]);
+            ss += cv[e] * cv[e];
+        }
+    }
+    ss = wave_sum_f32(ss);
+    if (lane == 0) red[wave] = ss;
+    lds_only_barrier();
+    float tot = red[0];
+#pragma unroll
+    for (int w = 1; w < kWaves; ++w) tot += red[w];
+    const float inv = 1.0f / sqrtf(tot / static_cast<float>(k) + in.eps);
+    if (tid < nchunk) {
+#pragma clang fp contract(off)
+        half8_t o, rs;
+#pragma unroll
+        for (int e = 0; e < 8; ++e) {
+            o[e] = static_cast<half_t>((cv[e] * inv) * static_cast<float>(nv[e]));
+            rs[e] = static_cast<half_t>(cv[e]);
+        }
+        store_half8(s_x + 8 * tid, o);
+        if (blockIdx.x == 0) store_half8(in.residual_out + 8 * tid, rs);
+    }
+    lds_only_barrier();
+    float acc[R];
+#pragma unroll
+    for (int r = 0; r < R; ++r) acc[r] = 0.0f;
+#pragma unroll
+    for (int u = 0; u < NC; ++u) {
+        const int c = lane + kWave * u;
+        if (c < nchunk) {
+            const half8_t xs = load_half8(s_x + 8 * c);
+#pragma unroll
+            for (int r = 0; r < R; ++r) acc[r] = dot8(wv[u][r], xs, acc[r]);
+        }
+    }
+    store_wave_rows<R, kSilu>(wave_multi_sum<R>(acc, lane), out, row0, m, lane);
 }
 
 // ---------------------------------------------------------------- argmax --
@@ -418,22 +627,33 @@ extern "C" int32_t grout_gemv_f16(const uint16_t* weight, const uint16_t* x, uin
     GROUT_REQUIRE(out != nullptr, GROUT_ERR_NULL_POINTER);
     GROUT_REQUIRE((reinterpret_cast<uintptr_t>(out) & 1u) == 0, GROUT_ERR_ALIGNMENT);
     GROUT_REQUIRE(m >= 1 && k >= 8 && k % 8 == 0 && k <= kGemvMaxK, GROUT_ERR_ARG);
+    const hipStream_t s = to_hip(stream);
+    const dim3 block(kGemvThreads);
+    auto grid = [&](int rows) { return dim3(static_cast<unsigned>((m + rows - 1) / rows)); };
+    if (k <= kGemvWaveMaxK) {
+        // Two rows a wavefront where that leaves at least 2 wavefronts per SIMD.
+        constexpr int kWaves = kGemvThreads / kWave;
+        if (m >= 4 * 1024) {
+            hipLaunchKernelGGL(gemv_wave_kernel<2>, grid(2 * kWaves), block, 0, s, weight, x, out, m, k, 0, NormIn{});
+        } else {
+            hipLaunchKernelGGL(gemv_wave_kernel<1>, grid(kWaves), block, 0, s, weight, x, out, m, k, 0, NormIn{});
+        }
+        return launch_status();
+    }
     // Rows per workgroup, measured on the Qwen3-32B token step: 2 for the
     // projections (qkv 10240, o_proj and down 5120 rows: 11.41 against 11.51
     // ms/token with 8 and 4), 8 only for vocabulary-sized outputs (lm_head at
     // 2 rows cost 0.1 ms more), 1 below 2048 rows so short outputs still
     // spread over the CUs.
-    const int rows = m >= 16 * 1024 ? 8 : m >= 2 * 1024 ? 2 : 1;
-    const unsigned blocks = static_cast<unsigned>((m + rows - 1) / rows);
-    const hipStream_t s = to_hip(stream);
-    const dim3 block(kGemvThreads);
     const size_t lds = static_cast<int64_t>(m) * k >= (int64_t{1} << 28) && k > 4096
                            ? gemv_reserve_lds(kGemvResident)
                            : 0;
-    switch (rows) {
-        case 8: hipLaunchKernelGGL(gemv_f16_kernel<8>, dim3(blocks), block, lds, s, weight, x, out, m, k); break;
-        case 2: hipLaunchKernelGGL(gemv_f16_kernel<2>, dim3(blocks), block, 0, s, weight, x, out, m, k); break;
-        default: hipLaunchKernelGGL(gemv_f16_kernel<1>, dim3(blocks), block, 0, s, weight, x, out, m, k); break;
+    if (m >= 16 * 1024) {
+        hipLaunchKernelGGL(gemv_f16_kernel<8>, grid(8), block, lds, s, weight, x, out, m, k);
+    } else if (m >= 2 * 1024) {
+        hipLaunchKernelGGL(gemv_f16_kernel<2>, grid(2), block, 0, s, weight, x, out, m, k);
+    } else {
+        hipLaunchKernelGGL(gemv_f16_kernel<1>, grid(1), block, 0, s, weight, x, out, m, k);
     }
     return launch_status();
 }
@@ -445,12 +665,57 @@ extern "C" int32_t grout_gemv_silu_mul_f16(const uint16_t* gate_up, const uint16
     GROUT_REQUIRE(out != nullptr, GROUT_ERR_NULL_POINTER);
     GROUT_REQUIRE((reinterpret_cast<uintptr_t>(out) & 1u) == 0, GROUT_ERR_ALIGNMENT);
     GROUT_REQUIRE(n >= 1 && n <= (1 << 29) && k >= 8 && k % 8 == 0 && k <= kGemvMaxK, GROUT_ERR_ARG);
+    if (k <= kGemvWaveMaxK) {
+        constexpr int kWaves = kGemvThreads / kWave;
+        hipLaunchKernelGGL((gemv_wave_kernel<2, true>), dim3(static_cast<unsigned>((n + kWaves - 1) / kWaves)),
+                           dim3(kGemvThreads), 0, to_hip(stream), gate_up, x, out, n, k, n, NormIn{});
+        return launch_status();
+    }
     // One gate row and its up row per workgroup (n workgroups), at full
     // residency: on the Qwen3-32B token step 11.30 ms/token against 11.41
     // with 4 + 4 rows and 11.44 with 2 + 2; capping the 2-row workgroups'
     // residency at 2 or 4 per CU measured 13.71 and 11.81.
     hipLaunchKernelGGL((gemv_f16_kernel<2, true>), dim3(static_cast<unsigned>(n)), dim3(kGemvThreads),
                        0, to_hip(stream), gate_up, x, out, n, k, n);
+    return launch_status();
+}
+
+bool grout::add_norm_gemv_fits(int32_t k) { return k <= kNormGemvMaxK; }
+
+int32_t grout::add_norm_gemv(const uint16_t* residual, const uint16_t* x, const uint16_t* norm_weight,
+                             uint16_t* residual_out, float eps, const uint16_t* weight, uint16_t* out, int32_t m,
+                             int32_t k, bool silu, grout_stream_t stream) {
+    GROUT_REQUIRE_PTR(residual);
+    GROUT_REQUIRE_PTR(x);
+    GROUT_REQUIRE_PTR(norm_weight);
+    GROUT_REQUIRE_PTR(residual_out);
+    GROUT_REQUIRE_PTR(weight);
+    GROUT_REQUIRE_PTR(out);
+    GROUT_REQUIRE(residual_out != residual && residual_out != x, GROUT_ERR_ARG);
+    GROUT_REQUIRE(eps >= 0.0f && eps < 1.0e30f, GROUT_ERR_ARG);
+    GROUT_REQUIRE(m >= 1 && m <= (1 << 29) && k >= 8 && k % 8 == 0 && k <= kNormGemvMaxK, GROUT_ERR_ARG);
+    const NormIn in = {residual, x, norm_weight, residual_out, eps};
+    const hipStream_t s = to_hip(stream);
+    // Rows per workgroup: one output per wavefront with SiLU (two rows), else two.
+    auto grid = [&](int threads) {
+        const int rows = (silu ? 1 : 2) * threads / kWave;
+        return dim3(static_cast<unsigned>((m + rows - 1) / rows));
+    };
+    if (k <= kGemvWaveMaxK) {
+        if (silu) {
+            hipLaunchKernelGGL((gemv_wave_kernel<2, true, true>), grid(kGemvThreads), dim3(kGemvThreads), 0, s, weight, x,
+                               out, m, k, m, in);
+        } else {
+            hipLaunchKernelGGL((gemv_wave_kernel<2, false, true>), grid(kGemvThreads), dim3(kGemvThreads), 0, s, weight, x,
+                               out, m, k, 0, in);
+        }
+    } else if (silu) {
+        hipLaunchKernelGGL((norm_gemv_kernel<2, true>), grid(kNormGemvThreads), dim3(kNormGemvThreads), 0, s, weight, out,
+                           in, m, k, m);
+    } else {
+        hipLaunchKernelGGL((norm_gemv_kernel<2, false>), grid(kNormGemvThreads), dim3(kNormGemvThreads), 0, s, weight, out,
+                           in, m, k, 0);
+    }
     return launch_status();
 }
 

@@ -18,6 +18,7 @@
 
 #include "abi_util.h"
 #include "common.h"
+#include "decode_layer.h"
 
 using namespace grout;
 
@@ -130,18 +131,26 @@ extern "C" int32_t grout_qwen3_decode_step(const grout_qwen3_model* model,
     uint32_t* block_idx = at<uint32_t>(ws, w.block_idx);
     const int32_t qkv_rows = M.head_dim * (M.num_q_heads + 2 * M.num_kv_heads);
     const int32_t attn_width = M.head_dim * M.num_q_heads;
+    const bool fold = add_norm_gemv_fits(M.hidden);
 
     // src/model.rs:3120-3149: embedding, then the plain RMSNorm of layer 0.
     st = grout_embed_rms_norm_decode(M.token, M.embed_tokens, M.vocab, M.layers[0].input_norm,
                                      normed, hidden, M.eps, M.hidden, stream);
     for (int32_t l = 0; st == GROUT_OK && l < M.num_layers; ++l) {
         const grout_qwen3_layer& L = M.layers[l];
-        if (l > 0) {  // :3151-3163 fold the previous layer's MLP residual in
-            st = grout_add_rms_norm_decode(hidden_after_attn, ff_down, L.input_norm, normed,
-                                           hidden, M.eps, M.hidden, stream);
-            if (st != GROUT_OK) break;
+        // :3170-3176, behind layer 0 with the previous layer's MLP residual and
+        // the input norm folded in (:3151-3163).
+        if (l > 0 && fold) {
+            st = add_norm_gemv(hidden_after_attn, ff_down, L.input_norm, hidden, M.eps, L.qkv_proj, qkv, qkv_rows,
+                               M.hidden, false, stream);
+        } else {
+            if (l > 0) {
+                st = grout_add_rms_norm_decode(hidden_after_attn, ff_down, L.input_norm, normed, hidden, M.eps,
+                                               M.hidden, stream);
+                if (st != GROUT_OK) break;
+            }
+            st = grout_gemv_f16(L.qkv_proj, normed, qkv, qkv_rows, M.hidden, stream);
         }
-        st = grout_gemv_f16(L.qkv_proj, normed, qkv, qkv_rows, M.hidden, stream);  // :3170-3176
         if (st != GROUT_OK) break;
         st = grout_attn_decode_fused(qkv, L.q_norm, L.k_norm, M.inv_freq, q_out, L.k_cache,
                                      L.v_cache, att_partial, lse_partial, attn_out, counters,
@@ -151,11 +160,16 @@ extern "C" int32_t grout_qwen3_decode_step(const grout_qwen3_model* model,
         if (st != GROUT_OK) break;
         st = grout_gemv_f16(L.o_proj, attn_out, attn_proj, M.hidden, attn_width, stream);
         if (st != GROUT_OK) break;  // :3505-3511
-        st = grout_add_rms_norm_decode(hidden, attn_proj, L.post_attn_norm, normed,
-                                       hidden_after_attn, M.eps, M.hidden, stream);
-        if (st != GROUT_OK) break;  // :3513-3526
-        // :3529-3535 gate_up GEMV and :3556-3565 SiLU * up, in one launch.
-        st = grout_gemv_silu_mul_f16(L.gate_up_proj, normed, ff, M.intermediate, M.hidden, stream);
+        // :3513-3526 add + norm; :3529-3535 gate_up GEMV and :3556-3565 SiLU * up.
+        if (fold) {
+            st = add_norm_gemv(hidden, attn_proj, L.post_attn_norm, hidden_after_attn, M.eps, L.gate_up_proj, ff,
+                               M.intermediate, M.hidden, true, stream);
+        } else {
+            st = grout_add_rms_norm_decode(hidden, attn_proj, L.post_attn_norm, normed, hidden_after_attn, M.eps,
+                                           M.hidden, stream);
+            if (st != GROUT_OK) break;
+            st = grout_gemv_silu_mul_f16(L.gate_up_proj, normed, ff, M.intermediate, M.hidden, stream);
+        }
         if (st != GROUT_OK) break;
         st = grout_gemv_f16(L.down_proj, ff, ff_down, M.hidden, M.intermediate, stream);
     }                               // :3568-3574

@@ -258,6 +258,49 @@ def test_token_step_qwen3_06b_shapes(gpu):
         runner.close()
 
 
+@pytest.mark.parametrize("hidden,inter,vocab", [
+    (8, 8, 9),          # one chunk a row; one wavefront with outputs past the end
+    (1016, 40, 515),    # one wavefront a row pair, a ragged second chunk column
+    (1024, 72, 4099),   # its longest rows; two rows a wavefront in lm_head, an odd last pair
+    (1032, 24, 100),    # rows normalised into LDS: 129 chunks of 512 threads, workgroups half empty
+    (2560, 520, 300),   # its longest rows
+    (2568, 64, 300),    # norm launches of their own
+])
+def test_token_step_hidden_sizes(gpu, hidden, inter, vocab):
+    """Two layers on both sides of the limits of the GEMV forms with the add +
+    RMSNorm folded in: logits, token and caches against the oracle, the second
+    step from the first one's caches."""
+    import torch
+    import grout_amd
+
+    m = qwen3_tiny_model(1800 + hidden, layers=2, hidden=hidden, hq=4, hkv=2, inter=inter, vocab=vocab,
+                         max_seq=64, filled=20)
+    ref = copy.deepcopy(m)
+    dm = _device_model(torch, m)
+    token = torch.tensor([vocab - 1], dtype=torch.int32, device="cuda")
+    position = torch.zeros((1,), dtype=torch.int32, device="cuda")
+    logits = torch.zeros((vocab,), dtype=torch.float16, device="cuda")
+    print(f"[qwen3 step] hidden {hidden} inter {inter} vocab {vocab}", flush=True)
+    runner = grout_amd.Qwen3DecodeRunner(
+        **dm, token=token, position=position, logits=logits, num_q_heads=4, num_kv_heads=2,
+        eps=m["eps"], qk_scale_f16_bits=m["qk_scale_f16_bits"], num_splits=2, block_n=32,
+        prime_position=20)
+    try:
+        tok = vocab - 1
+        for pos in (20, 21):
+            if pos > 20:
+                runner.step(pos)
+            torch.cuda.synchronize()
+            rl, _ = oracle.qwen3_decode_step(ref, tok, pos, 32, 2, fused_ranges=True)
+            gl = logits.cpu().numpy()
+            assert_close_attn(gl, rl, f"hidden {hidden} position {pos} logits", atol=1e-2, rtol=1e-2)
+            tok = int(token.item())
+            assert tok == oracle.argmax_f16(gl)
+        _check_caches(dm, ref, [20, 21])
+    finally:
+        runner.close()
+
+
 def test_runner_step_after_eager_step_writes_position(gpu):
     """step(p), an eager step (which moves the device position to p+2), then
     step(p+1): the replay runs at p+1, as launch_step writes the position on
