@@ -75,6 +75,15 @@ def _ensure(cond: bool, msg: str):
         raise GroutError(msg)
 
 
+# The launches of single ops take less GPU time than a careless wrapper takes
+# host time (a 37-token prompt: 9 us of kernels, 28 us for its two calls).  Their
+# checks are written ``if not ...: _fail(f"...")``, so that a message with its
+# shape lists is only formatted when the check fails, and look the stream up
+# without building a Stream object.
+def _fail(msg: str):
+    raise GroutError(msg)
+
+
 def _torch():
     import torch
     return torch
@@ -86,6 +95,8 @@ def _ptr(t) -> int:
 
 def _stream() -> int:
     torch = _torch()
+    if torch.cuda.is_initialized():
+        return torch._C._cuda_getCurrentRawStream(torch._C._cuda_getDevice())
     return torch.cuda.current_stream().cuda_stream
 
 
@@ -94,6 +105,14 @@ def _f16(t, name: str):
     _ensure(t.dtype == torch.float16, f"{name} must be f16, got {t.dtype}")
     _ensure(t.is_cuda, f"{name} must be a device tensor")
     _ensure(t.is_contiguous(), f"{name} must be contiguous")
+
+
+def _all_f16(*named):
+    """_f16 of each (tensor, name), in order."""
+    f16 = _torch().float16
+    for t, name in named:
+        if t.dtype is not f16 or not t.is_cuda or not t.is_contiguous():
+            _f16(t, name)
 
 
 def build_inv_freq(theta: float, head_dim: int = HEAD_DIM):
@@ -110,27 +129,28 @@ def qk_norm_rope_kv_prefill(q, k, v, q_weight, k_weight, inv_freq, out, k_cache,
 
     q [S,Hq,D], k/v [S,Hkv,D], out [S,Hq,D]; writes cache rows
     [position_start, position_start+S) of k_cache/v_cache [Hkv,MS,D]."""
-    _ensure(q.dim() == 3, f"q shape mismatch in fused qk/rope/kv prefill: {list(q.shape)}")
+    if q.dim() != 3:
+        _fail(f"q shape mismatch in fused qk/rope/kv prefill: {list(q.shape)}")
     S, Hq, D = q.shape
-    _ensure(k.dim() == 3 and k.shape[0] == S and k.shape[2] == D,
-            f"k shape mismatch in fused qk/rope/kv prefill: {list(k.shape)}")
+    if k.dim() != 3 or k.shape[0] != S or k.shape[2] != D:
+        _fail(f"k shape mismatch in fused qk/rope/kv prefill: {list(k.shape)}")
     Hkv = k.shape[1]
-    _ensure(list(v.shape) == [S, Hkv, D],
-            f"v shape mismatch in fused qk/rope/kv prefill: {list(v.shape)}")
-    _ensure(list(out.shape) == [S, Hq, D],
-            f"fused qk/rope/kv output shape mismatch: {list(out.shape)}")
-    _ensure(D % 2 == 0, f"fused qk/rope/kv requires even head_dim, got {D}")
+    if v.shape != (S, Hkv, D):
+        _fail(f"v shape mismatch in fused qk/rope/kv prefill: {list(v.shape)}")
+    if out.shape != (S, Hq, D):
+        _fail(f"fused qk/rope/kv output shape mismatch: {list(out.shape)}")
+    if D % 2 != 0:
+        _fail(f"fused qk/rope/kv requires even head_dim, got {D}")
     MS = k_cache.shape[1] if k_cache.dim() == 3 else -1
-    _ensure(position_start + S <= MS,
-            f"fused qk/rope/kv range [{position_start}..{position_start + S}) exceeds "
-            f"max_seq_len {MS}")
-    _ensure(list(k_cache.shape) == [Hkv, MS, D],
-            f"k_cache shape mismatch in fused qk/rope/kv: {list(k_cache.shape)}")
-    _ensure(list(v_cache.shape) == [Hkv, MS, D],
-            f"v_cache shape mismatch in fused qk/rope/kv: {list(v_cache.shape)}")
-    for t, n in ((q, "q"), (k, "k"), (v, "v"), (q_weight, "q_weight"), (k_weight, "k_weight"),
-                 (out, "out"), (k_cache, "k_cache"), (v_cache, "v_cache")):
-        _f16(t, n)
+    if position_start + S > MS:
+        _fail(f"fused qk/rope/kv range [{position_start}..{position_start + S}) exceeds "
+              f"max_seq_len {MS}")
+    if k_cache.shape != (Hkv, MS, D):
+        _fail(f"k_cache shape mismatch in fused qk/rope/kv: {list(k_cache.shape)}")
+    if v_cache.shape != (Hkv, MS, D):
+        _fail(f"v_cache shape mismatch in fused qk/rope/kv: {list(v_cache.shape)}")
+    _all_f16((q, "q"), (k, "k"), (v, "v"), (q_weight, "q_weight"), (k_weight, "k_weight"),
+             (out, "out"), (k_cache, "k_cache"), (v_cache, "v_cache"))
     _check(lib().grout_qk_norm_rope_kv_prefill(
         _ptr(q), _ptr(k), _ptr(v), _ptr(q_weight), _ptr(k_weight), _ptr(inv_freq), _ptr(out),
         _ptr(k_cache), _ptr(v_cache), float(eps), int(position_start), S, Hq, Hkv, D, MS,
@@ -141,17 +161,17 @@ def qk_norm_rope_kv_prefill(q, k, v, q_weight, k_weight, inv_freq, out, k_cache,
 def _kv_update_checks(new_k, new_v, k_cache, v_cache):
     """The shape ensure!s of kv_cache_update_seq_arc_ctx_with_position
     (src/model.rs:5396-5423); returns (S, Hkv, D, MS)."""
-    _ensure(new_k.dim() == 3,
-            f"new_k must be rank 3 [seqlen, kv_heads, head_dim], got {list(new_k.shape)}")
+    if new_k.dim() != 3:
+        _fail(f"new_k must be rank 3 [seqlen, kv_heads, head_dim], got {list(new_k.shape)}")
     S, Hkv, D = new_k.shape
-    _ensure(k_cache.dim() == 3 and k_cache.shape[0] == Hkv and k_cache.shape[2] == D,
-            f"new_k shape mismatch: {list(new_k.shape)}")
-    _ensure(list(new_v.shape) == [S, Hkv, D], f"new_v shape mismatch: {list(new_v.shape)}")
+    if k_cache.dim() != 3 or k_cache.shape[0] != Hkv or k_cache.shape[2] != D:
+        _fail(f"new_k shape mismatch: {list(new_k.shape)}")
+    if new_v.shape != (S, Hkv, D):
+        _fail(f"new_v shape mismatch: {list(new_v.shape)}")
     MS = k_cache.shape[1]
-    _ensure(list(v_cache.shape) == [Hkv, MS, D],
-            f"v_cache shape mismatch: {list(v_cache.shape)}")
-    for t, n in ((new_k, "new_k"), (new_v, "new_v"), (k_cache, "k_cache"), (v_cache, "v_cache")):
-        _f16(t, n)
+    if v_cache.shape != (Hkv, MS, D):
+        _fail(f"v_cache shape mismatch: {list(v_cache.shape)}")
+    _all_f16((new_k, "new_k"), (new_v, "new_v"), (k_cache, "k_cache"), (v_cache, "v_cache"))
     return S, Hkv, D, MS
 
 
@@ -160,9 +180,9 @@ def kv_cache_update_seq(new_k, new_v, k_cache, v_cache, position_start: int):
     (src/model.rs:5388-5480, kv_cache_update_seq_f16): cache rows
     [position_start, position_start+S) of every KV head take new_k/new_v."""
     S, Hkv, D, MS = _kv_update_checks(new_k, new_v, k_cache, v_cache)
-    _ensure(position_start + S <= MS,
-            f"kv_cache_update range [{position_start}..{position_start + S}) exceeds "
-            f"max_seq_len {MS}")
+    if position_start + S > MS:
+        _fail(f"kv_cache_update range [{position_start}..{position_start + S}) exceeds "
+              f"max_seq_len {MS}")
     _check(lib().grout_kv_cache_update_seq(
         _ptr(new_k), _ptr(new_v), _ptr(k_cache), _ptr(v_cache), int(position_start), S, Hkv, D,
         MS, _stream()), "kv_cache_update_seq")
@@ -210,25 +230,25 @@ def attend_prefill(q, k_cache, v_cache, out, position_start: int,
     is bit-identical to the static grid's.  A few rows behind many keys take
     grout_attn_prefill_ws with scratch from torch's allocator, except while the
     current stream is being captured."""
-    _ensure(q.dim() == 3, f"q must be rank 3 [seqlen, heads, head_dim], got {list(q.shape)}")
+    if q.dim() != 3:
+        _fail(f"q must be rank 3 [seqlen, heads, head_dim], got {list(q.shape)}")
     q_len, Hq, D = q.shape
     Hkv, MS, _ = k_cache.shape
-    _ensure(list(out.shape) == [q_len, Hq, D],
-            f"attend output shape mismatch, got {list(out.shape)}")
+    if out.shape != (q_len, Hq, D):
+        _fail(f"attend output shape mismatch, got {list(out.shape)}")
     if qk_scale is None:
         qk_scale = 1.0 / math.sqrt(float(D))
     if kv_len is None:
         kv_len = position_start + q_len
-    for t, n in ((q, "q"), (k_cache, "k_cache"), (v_cache, "v_cache"), (out, "out")):
-        _f16(t, n)
+    _all_f16((q, "q"), (k_cache, "k_cache"), (v_cache, "v_cache"), (out, "out"))
     args = (_ptr(q), _ptr(k_cache), _ptr(v_cache), _ptr(out), float(qk_scale), Hq, Hkv, D, q_len,
             int(kv_len), int(position_start), MS)
     if sched_counters is not None:
-        _ensure(sched_counters.is_cuda and sched_counters.is_contiguous(),
-                "sched_counters must be a contiguous device tensor")
-        _ensure(sched_counters.numel() * sched_counters.element_size()
-                >= lib().grout_attn_prefill_sched_counter_bytes(),
-                "sched_counters is smaller than grout_attn_prefill_sched_counter_bytes()")
+        if not (sched_counters.is_cuda and sched_counters.is_contiguous()):
+            _fail("sched_counters must be a contiguous device tensor")
+        if (sched_counters.numel() * sched_counters.element_size()
+                < lib().grout_attn_prefill_sched_counter_bytes()):
+            _fail("sched_counters is smaller than grout_attn_prefill_sched_counter_bytes()")
     workspace = None
     if kv_len > 512:  # shorter key ranges never split
         workspace = _prefill_workspace(q.device, Hq, Hkv, D, q_len, int(kv_len), int(position_start), MS)
@@ -333,9 +353,9 @@ def add_rms_norm_decode(residual, x, weight, out, residual_out, eps: float):
     args = ((residual, "residual"), (x, "x"), (weight, "weight"), (out, "out"),
             (residual_out, "residual_out"))
     for t, nm in args:
-        _ensure(t.numel() == n, f"{nm} must have {n} elements, got {t.numel()}")
-    for t, nm in args:
-        _f16(t, nm)
+        if t.numel() != n:
+            _fail(f"{nm} must have {n} elements, got {t.numel()}")
+    _all_f16(*args)
     _check(lib().grout_add_rms_norm_decode(_ptr(residual), _ptr(x), _ptr(weight), _ptr(out),
                                            _ptr(residual_out), float(eps), n, _stream()),
            "add_rms_norm_decode")
@@ -344,12 +364,14 @@ def add_rms_norm_decode(residual, x, weight, out, residual_out, eps: float):
 
 def gemv_f16(weight, x, out):
     """cuBLAS GemvInPlace (src/cublas.rs:572-607): out[m] = weight[m, k] @ x[k], f32 accumulate."""
-    _ensure(weight.dim() == 2, f"weight must be [m, k], got {list(weight.shape)}")
+    if weight.dim() != 2:
+        _fail(f"weight must be [m, k], got {list(weight.shape)}")
     m, k = weight.shape
-    _ensure(x.numel() == k, f"x must have {k} elements, got {x.numel()}")
-    _ensure(out.numel() == m, f"out must have {m} elements, got {out.numel()}")
-    for t, nm in ((weight, "weight"), (x, "x"), (out, "out")):
-        _f16(t, nm)
+    if x.numel() != k:
+        _fail(f"x must have {k} elements, got {x.numel()}")
+    if out.numel() != m:
+        _fail(f"out must have {m} elements, got {out.numel()}")
+    _all_f16((weight, "weight"), (x, "x"), (out, "out"))
     _check(lib().grout_gemv_f16(_ptr(weight), _ptr(x), _ptr(out), m, k, _stream()), "gemv_f16")
     return out
 
@@ -358,13 +380,14 @@ def gemv_silu_mul(gate_up, x, out):
     """The gate_up GEMV and silu_mul_2d_f16 of the decode graph (src/model.rs:3529-3535,
     3556-3565) in one launch: out[n] = silu(gate) * up of the f16 rows of gate_up[2n, k] @ x,
     bit-identical to gemv_f16 followed by silu_mul."""
-    _ensure(gate_up.dim() == 2 and gate_up.shape[0] % 2 == 0,
-            f"gate_up must be [2n, k], got {list(gate_up.shape)}")
+    if gate_up.dim() != 2 or gate_up.shape[0] % 2 != 0:
+        _fail(f"gate_up must be [2n, k], got {list(gate_up.shape)}")
     m2, k = gate_up.shape
-    _ensure(x.numel() == k, f"x must have {k} elements, got {x.numel()}")
-    _ensure(out.numel() == m2 // 2, f"out must have {m2 // 2} elements, got {out.numel()}")
-    for t, nm in ((gate_up, "gate_up"), (x, "x"), (out, "out")):
-        _f16(t, nm)
+    if x.numel() != k:
+        _fail(f"x must have {k} elements, got {x.numel()}")
+    if out.numel() != m2 // 2:
+        _fail(f"out must have {m2 // 2} elements, got {out.numel()}")
+    _all_f16((gate_up, "gate_up"), (x, "x"), (out, "out"))
     _check(lib().grout_gemv_silu_mul_f16(_ptr(gate_up), _ptr(x), _ptr(out), m2 // 2, k, _stream()),
            "gemv_silu_mul_f16")
     return out
@@ -569,12 +592,15 @@ def decode_fused(qkv, q_weight, k_weight, inv_freq, q_out, k_cache, v_cache, att
     [Hkv, G, D]; with advance_position the device position ends one higher."""
     D = q_weight.shape[0]
     G = num_q_heads // num_kv_heads
-    _ensure(qkv.numel() == (num_q_heads + 2 * num_kv_heads) * D, "qkv size mismatch")
-    _ensure(att_partial.dim() == 3 and att_partial.shape[1] % G == 0, "att_partial shape mismatch")
+    if qkv.numel() != (num_q_heads + 2 * num_kv_heads) * D:
+        _fail("qkv size mismatch")
+    if att_partial.dim() != 3 or att_partial.shape[1] % G != 0:
+        _fail("att_partial shape mismatch")
     ns = att_partial.shape[1] // G
-    _ensure(counters.numel() * 4 >= lib().grout_attn_decode_counter_bytes(num_kv_heads),
-            "counters too small")
-    _check(lib().grout_attn_decode_fused(
+    L = lib()
+    if counters.numel() * 4 < L.grout_attn_decode_counter_bytes(num_kv_heads):
+        _fail("counters too small")
+    _check(L.grout_attn_decode_fused(
         _ptr(qkv), _ptr(q_weight), _ptr(k_weight), _ptr(inv_freq), _ptr(q_out), _ptr(k_cache),
         _ptr(v_cache), _ptr(att_partial), _ptr(lse_partial), _ptr(out), _ptr(counters),
         _ptr(position), float(eps), int(qk_scale_f16_bits), num_q_heads, num_kv_heads, D,
