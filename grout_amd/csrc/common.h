@@ -17,6 +17,8 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include <type_traits>
+
 namespace grout {
 
 typedef _Float16 half_t;
@@ -78,6 +80,59 @@ __device__ __forceinline__ float swap_rows16(float x) {
     auto r = __builtin_amdgcn_permlane16_swap(xi, xi, false, false);
     int lane = __lane_id();
     return __builtin_bit_cast(float, (lane & 16) ? (int)r[0] : (int)r[1]);
+}
+
+// Value of lane l ^ 1, l ^ 2, and the sum over each aligned group of 8 lanes by
+// DPP moves (quad swaps, then the mirror of 8, which pairs quads that already
+// hold their sums): the adds of three xor shuffles, without their LDS trips.
+__device__ __forceinline__ float sum8_dpp(float x) {
+    const auto move = [](float v, auto ctrl) {
+        return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v),
+                                                                     decltype(ctrl)::value, 0xf, 0xf, false));
+    };
+    x += move(x, std::integral_constant<int, 0xB1>{});   // quad_perm [1,0,3,2]
+    x += move(x, std::integral_constant<int, 0x4E>{});   // quad_perm [2,3,0,1]
+    x += move(x, std::integral_constant<int, 0x141>{});  // row_half_mirror
+    return x;
+}
+
+constexpr double inv_factorial_of(int n) { return n <= 1 ? 1.0 : inv_factorial_of(n - 1) / n; }
+template <int n>
+constexpr double kInvFact = inv_factorial_of(n);
+
+// sin and cos of an f32 angle, each rounded once to f32 from an f64 value good
+// to ~1e-16.  theta = n pi/2 + r with |r| <= pi/4: pi/2's f64 value is a multiple
+// of 2^-52, so x - n hi is exact in one FMA, and the second FMA takes n times the
+// rest of pi/2.  Taylor series in r^2 to r^17 and r^16 (the terms left out are
+// below 2e-18), summed pairwise: a launch waits for one such chain, and the
+// library's sincos is ~1600 cycles long.  Angles of 2^30 and more, infinities and
+// NaN take the library's.
+__device__ __forceinline__ void sincos_f32(float theta, float* sn, float* cs) {
+    const double x = static_cast<double>(theta);
+    double sv, cv;
+    if (__builtin_expect(fabsf(theta) < 1073741824.0f, 1)) {
+        constexpr double kTwoOverPi = 0.63661977236758134308;
+        constexpr double kPio2Hi = 1.57079632679489655800;
+        constexpr double kPio2Lo = 6.12323399573676603587e-17;
+        const double n = __builtin_rint(x * kTwoOverPi);
+        const double r = fma(-n, kPio2Lo, fma(-n, kPio2Hi, x));
+        const int q = static_cast<int>(n);
+        const double z = r * r, z2 = z * z, z4 = z2 * z2;
+        const double p = fma(z4, fma(z2, fma(kInvFact<17>, z, -kInvFact<15>), fma(kInvFact<13>, z, -kInvFact<11>)),
+                             fma(z2, fma(kInvFact<9>, z, -kInvFact<7>), fma(kInvFact<5>, z, -kInvFact<3>)));
+        const double c = fma(z4, fma(z2, kInvFact<16>, fma(-kInvFact<14>, z, kInvFact<12>)),
+                             fma(z2, fma(-kInvFact<10>, z, kInvFact<8>), fma(-kInvFact<6>, z, kInvFact<4>)));
+        const double sr = fma(r * z, p, r);
+        const double cr = fma(z2, c, fma(-0.5, z, 1.0));
+        sv = (q & 1) ? cr : sr;
+        cv = (q & 1) ? sr : cr;
+        if (q & 2) sv = -sv;
+        if ((q + 1) & 2) cv = -cv;
+    } else {
+        sincos(x, &sv, &cv);
+    }
+    *sn = static_cast<float>(sv);
+    *cs = static_cast<float>(cv);
 }
 
 // Orders LDS traffic of one wavefront (lanes exchange data through LDS

@@ -11,7 +11,7 @@
 //  * Eight lanes own one 128-wide head row: lane t holds elements
 //    [8t, 8t+8) of the low half and [64+8t, 64+8t+8) of the high half, so
 //    each RoPE pair (j, j+64) sits in one lane and every access is 16 bytes.
-//  * The row's sum of squares is reduced over the 8 lanes with xor shuffles.
+//  * The row's sum of squares is reduced over the 8 lanes with DPP moves.
 // Arithmetic follows the reference order: ss = sum(lo*lo + hi*hi),
 // inv = 1/sqrt(ss/128 + eps), n = x*inv*w, y_lo = n_lo*cos - n_hi*sin,
 // y_hi = n_hi*cos + n_lo*sin, f16 round-to-nearest-even.  Contraction into
@@ -71,10 +71,7 @@ __global__ __launch_bounds__(kNormThreads) void qk_norm_rope_kv_kernel(
     for (int i = tid; i < ntok * 64; i += kNormThreads) {
         const int t = i >> 6, j = i & 63;
         const float theta = static_cast<float>(pos0 + t) * inv_freq[j];
-        double sv, cv;
-        sincos(static_cast<double>(theta), &sv, &cv);
-        s_cos[t][j] = static_cast<float>(cv);
-        s_sin[t][j] = static_cast<float>(sv);
+        sincos_f32(theta, &s_sin[t][j], &s_cos[t][j]);
     }
     __syncthreads();
 
@@ -104,9 +101,7 @@ __global__ __launch_bounds__(kNormThreads) void qk_norm_rope_kv_kernel(
             const float b = static_cast<float>(xhi[i]);
             ss += a * a + b * b;
         }
-        ss += __shfl_xor(ss, 1);
-        ss += __shfl_xor(ss, 2);
-        ss += __shfl_xor(ss, 4);
+        ss = sum8_dpp(ss);
         const float inv_rms = 1.0f / sqrtf(ss / 128.0f + eps);
 
         half8_t ylo, yhi;

@@ -167,3 +167,33 @@ def test_decode_equals_prefill_row(gpu):
     torch.cuda.synchronize()
     assert torch.equal(qo1[:hq], qo2[0])
     assert torch.equal(kc1, kc2) and torch.equal(vc1, vc2)
+
+
+@pytest.mark.parametrize("scale,start", [
+    (1.0, 0), (1.0, 40000),   # angles up to 4e4 and below 1e-2
+    (3.0e4, 35700),           # past 2^30: the large-angle path for some frequencies
+    (1.0e25, 35700),          # all of them
+])
+def test_angles_correctly_rounded(gpu, scale, start):
+    """cos and sin of the f32 angles, read back through the op: a row of ones
+    under weight ones gives cos - sin and cos + sin of each frequency, here held
+    to float64 within f16 rounding (half an ulp, plus the f32 roundings of the two
+    factors and the sum: 1.5 * 2^-23 of values up to 1)."""
+    import torch
+    import grout_amd
+
+    S = 33
+    inv = grout_amd.build_inv_freq(1e6) * scale
+    ones = torch.ones((S, 1, 128), dtype=torch.float16, device="cuda")
+    w = torch.ones((128,), dtype=torch.float16, device="cuda")
+    out = torch.empty_like(ones)
+    cache = torch.zeros((1, start + S, 128), dtype=torch.float16, device="cuda")
+    print(f"[rope angles] scale {scale} start {start}", flush=True)
+    grout_amd.qk_norm_rope_kv_prefill(ones, ones, ones, w, w, inv.cuda(), out, cache, cache.clone(), 0.0, start)
+    got = out[:, 0].double().cpu()
+    pos = torch.arange(start, start + S, dtype=torch.float32)
+    theta = (pos[:, None] * inv[None, :]).numpy().astype(np.float64)
+    c, s = torch.from_numpy(np.cos(theta)), torch.from_numpy(np.sin(theta))
+    ref = torch.cat([c - s, c + s], dim=1)
+    ulp = torch.clamp(2.0 ** (torch.floor(torch.log2(ref.abs().clamp_min(2.0 ** -14))) - 10), min=2.0 ** -24)
+    assert bool(((got - ref).abs() <= 0.5 * ulp + 1.5 * 2.0 ** -23).all())
