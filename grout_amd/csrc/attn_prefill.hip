@@ -255,11 +255,15 @@ __device__ __forceinline__ void pf_gemm_half(const unsigned char* kb, const unsi
 // Softmax of one (already masked) tile: P = 2^(c*s - m) into `pop`, its row
 // sum into l, with the running max m raised only when it has to be.
 // kBlocks: 32-key blocks of the tile (2: the grid's 64 keys, 1: half a tile).
-template <int kBlocks>
+// fill(i), i < 8 kBlocks, runs before the i-th pair of exponentials.
+struct NoFill {
+    __device__ __forceinline__ void operator()(int) const {}
+};
+template <int kBlocks, typename Fill = NoFill>
 __device__ __forceinline__ void pf_softmax(const float16_t (&s)[kBlocks], half8_t (&pop)[2 * kBlocks],
-                                           float16_t (&o)[4], float& m_run, float& l_run, float c) {
+                                           float16_t (&o)[4], float& m_run, float& l_run, float c, Fill fill = Fill{}) {
     // The row sum runs in four independent f32 chains.
-    auto exp_tile = [&](float m_use) {
+    auto exp_tile = [&](float m_use, auto filler) {
         // Each chain starts from its first pair rather than from 0.0f: the
         // compiler keeps a float 0 + x (it is not x for x = -0), and those
         // four adds measured ~1% of the kernel's time.  p >= 0, so the
@@ -269,6 +273,7 @@ __device__ __forceinline__ void pf_softmax(const float16_t (&s)[kBlocks], half8_
         for (int mb = 0; mb < kBlocks; ++mb)
 #pragma unroll
             for (int r = 0; r < 16; r += 2) {
+                filler(8 * mb + (r >> 1));
                 const float p0 = __builtin_amdgcn_exp2f(fmaf(s[mb][r], c, -m_use));
                 const float p1 = __builtin_amdgcn_exp2f(fmaf(s[mb][r + 1], c, -m_use));
                 const int k = (r >> 1) & 3;
@@ -278,7 +283,7 @@ __device__ __forceinline__ void pf_softmax(const float16_t (&s)[kBlocks], half8_
             }
         return (ps[0] + ps[1]) + (ps[2] + ps[3]);
     };
-    float psum = exp_tile(m_run);
+    float psum = exp_tile(m_run, fill);
     // The max is only raised when P would leave f16 range: a lane's partial
     // row sum below 2^15 bounds each of its p below 2^15 (the test also
     // catches inf).  Then the tile's row max becomes the running max, O and
@@ -297,9 +302,39 @@ __device__ __forceinline__ void pf_softmax(const float16_t (&s)[kBlocks], half8_
 #pragma unroll
         for (int db = 0; db < 4; ++db) o[db] *= alpha;
         m_run = m_new;
-        psum = exp_tile(m_run);
+        psum = exp_tile(m_run, NoFill{});
     }
     l_run += psum;
+}
+
+// S^T = K Q^T of one tile alone (`kb`: this lane's base in its K stage).
+__device__ __forceinline__ void pf_scores(const unsigned char* kb, const half8_t (&qop)[8], float16_t (&s)[2]) {
+#pragma unroll
+    for (int mb = 0; mb < 2; ++mb)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) s[mb][r] = 0.0f;
+#pragma unroll
+    for (int i = 0; i < 16; ++i)
+        s[i & 1] = mfma32x32x16(*reinterpret_cast<const half8_t*>(kb + 512 * (i & 1) + 32 * (i >> 1)), qop[i >> 1], s[i & 1]);
+}
+
+// O^T += V^T P^T of one tile alone (`vb`: this lane's base in its V stage).
+__device__ __forceinline__ void pf_values(const unsigned char* vb, const half8_t (&pop)[4], float16_t (&o)[4]) {
+    constexpr int kRing = kPfAhead + 1;
+    auto read_op = [&](int i) {
+        const unsigned char* p0 = vb + 256 * (i >> 2) + 64 * (i & 3);
+        return cat(lds_read_tr16(reinterpret_cast<const half_t*>(p0)),
+                   lds_read_tr16(reinterpret_cast<const half_t*>(p0 + 8 * kPfVBlock)));
+    };
+    half8_t ring[kRing];
+#pragma unroll
+    for (int i = 0; i < kPfAhead; ++i) ring[i % kRing] = read_op(i);
+#pragma unroll
+    for (int i = 0; i < 16; ++i) {
+        if (i + kPfAhead < 16) ring[(i + kPfAhead) % kRing] = read_op(i + kPfAhead);
+        o[i & 3] = mfma32x32x16(ring[i % kRing], pop[i >> 2], o[i & 3]);
+        __builtin_amdgcn_sched_barrier(0);
+    }
 }
 
 // Workgroup: 8 wavefronts x 32 query rows, all on query heads of one KV head.
@@ -326,8 +361,14 @@ constexpr int kPfRows = 32;
 // small to fill the GPU: twice the workgroups, and a tile step takes one GEMM
 // phase and one softmax phase.  A 1 KB copy holds up the wavefront that issues
 // it for ~100 cycles; left to the computing wavefronts, their eight copies a
-// step were ~800 of ~2850 cycles, with the copy wavefronts a step takes ~2300
+// step were ~800 of ~2850 cycles, with the copy wavefronts a step took ~2300
 // (Qwen3-4B, 1000 tokens 24.3 -> 21.3 us; 509 tokens behind 6003 117 -> 95 us).
+// Without a partner to alternate with, a step computes S of the next tile
+// between the exponentials of this one, then this one's PV: ~2090 cycles (Qwen3-0.6B,
+// 927 tokens 19.0 -> 17.8 us; 32/8 heads, 768 behind 4096 73.3 -> 71.7).  Of
+// these 1390 are the softmax with its 16 S MFMAs and 620 PV: one wavefront's
+// MFMAs and VALU hardly overlap, and spreading the softmax over PV's MFMAs of
+// the tile before as well measured the same.
 // Every wavefront computes exactly what it computes in the 8-wavefront
 // workgroup, so the output is bit-identical.
 template <bool kSplit, bool kDyn, int kWaves = kPfWaves>
@@ -647,8 +688,7 @@ __global__ __launch_bounds__(kPfWaves * kWave, 1) void attn_prefill_kernel(Prefi
     // O = 0, LSE = -1e30, weight 0 in the merge (the reference's -1e30 gives
     // such rows p = 1 and an LSE near -1.3e29: also weight 0).
     constexpr float kMasked = kSplit ? -__builtin_inff() : kPfNegBig;
-    auto softmax_phase = [&](int j) {
-        if (j < wave_t0 || j >= wave_tiles) return;
+    auto mask_tile = [&](int j, float16_t (&sc)[2]) {
         const int n0 = (tile0 + j) * kPfBN;
         bool need_mask = (n0 + kPfBN - 1 > pos0) || (n0 + kPfBN > a.kv_len);
         if constexpr (kSplit) need_mask = need_mask || n0 < key_lo || n0 + kPfBN > key_hi;
@@ -663,9 +703,13 @@ __global__ __launch_bounds__(kPfWaves * kWave, 1) void attn_prefill_kernel(Prefi
 #pragma unroll
                 for (int r = 0; r < 16; ++r) {
                     const int rel = rel0 + 32 * mb + 8 * (r >> 2) + (r & 3);
-                    if (static_cast<uint32_t>(rel) >= span) s[mb][r] = kMasked;
+                    if (static_cast<uint32_t>(rel) >= span) sc[mb][r] = kMasked;
                 }
         }
+    };
+    auto softmax_phase = [&](int j) {
+        if (j < wave_t0 || j >= wave_tiles) return;
+        mask_tile(j, s);
         pf_softmax<2>(s, pop, o, m_run, l_run, c);
     };
 
@@ -685,11 +729,52 @@ __global__ __launch_bounds__(kPfWaves * kWave, 1) void attn_prefill_kernel(Prefi
     // start of the step.  Issued by all eight wavefronts right after the
     // barrier, the copies queue behind each other and hold up the GEMM phase
     // of group A (measured ~1% slower, bit-identical output).
-    if (kWaves == 4 || grp == 0) {
+    if constexpr (kWaves == 4) {
+        // One wavefront per SIMD: S of tile t+1 runs under the softmax of tile
+        // t (an S MFMA before every pair of exponentials), then PV of tile t.
+        // The barrier before step t opens tile t+1; tile t+3 goes into the
+        // stage of tile t-1, whose PV ended before it.  Two score buffers
+        // alternate.
+        auto k_base = [&](int j) { return pf_lds + (j % kPfStages) * kPfStageBytes + k_lane; };
+        auto step = [&](int t, float16_t (&cur)[2], float16_t (&nxt)[2]) {
+            pf_barrier();
+            if (t >= wave_tiles) return;
+            mask_tile(t, cur);
+            if (t + 1 < wave_tiles) {
+                const unsigned char* kb = k_base(t + 1);
+                constexpr int kRing = kPfAhead + 1;
+                half8_t ring[kRing];
+                auto read_op = [&](int i) {
+                    return *reinterpret_cast<const half8_t*>(kb + 512 * (i & 1) + 32 * (i >> 1));
+                };
+#pragma unroll
+                for (int mb = 0; mb < 2; ++mb)
+#pragma unroll
+                    for (int r = 0; r < 16; ++r) nxt[mb][r] = 0.0f;
+#pragma unroll
+                for (int i = 0; i < kPfAhead; ++i) ring[i % kRing] = read_op(i);
+                pf_softmax<2>(cur, pop, o, m_run, l_run, c, [&](int i) {
+                    if (i + kPfAhead < 16) ring[(i + kPfAhead) % kRing] = read_op(i + kPfAhead);
+                    nxt[i & 1] = mfma32x32x16(ring[i % kRing], qop[i >> 1], nxt[i & 1]);
+                    __builtin_amdgcn_sched_barrier(0);
+                });
+            } else {
+                pf_softmax<2>(cur, pop, o, m_run, l_run, c);
+            }
+            pf_values(pf_lds + (t % kPfStages) * kPfStageBytes + kPfKBytes + v_lane, pop, o);
+        };
+        float16_t s2[2];
+        pf_barrier();
+        if (wave_tiles > 0) pf_scores(k_base(0), qop, s);
+        for (int t = 0; t < ntiles; t += 2) {
+            step(t, s, s2);
+            if (t + 1 < ntiles) step(t + 1, s2, s);
+        }
+    } else if (grp == 0) {
         for (int t = 0; t <= ntiles; ++t) {
             open_tile_step(t);
             gemm_phase(t);
-            if (kWaves != 4 && t + 2 < ntiles) issue_tile(t + 2, (t + 2) % kPfStages, std::false_type{});
+            if (t + 2 < ntiles) issue_tile(t + 2, (t + 2) % kPfStages, std::false_type{});
             softmax_phase(t);
         }
     } else {
@@ -1368,11 +1453,12 @@ static int64_t prefill_rounds(int64_t blocks, int64_t cus, int64_t most, int64_t
 }
 
 // Whether 4-tile workgroups (blocks4) beat 8-tile ones (blocks8).  A step of
-// the former takes 4/5 of a step of the latter (0.96 against 1.22 us), so they
-// lose once the grid needs as many rounds of workgroups more.  Measured, 4 against 8
-// tiles: 32/8 heads 1500 tokens 28.7 / 35.8 us, 2048 45.0 / 50.1, 3000 93.9 /
-// 82.0; 64/8 heads 1024 tokens 27.6 / 29.9, 2048 88.3 / 73.5; 16/8 heads 4096
-// tokens 79.8 / 90.8; 32/8 heads, 1024 tokens behind 8192, 157 / 168.
+// the former takes about 4/5 of a step of the latter (0.92 against 1.22 us), so
+// they lose once the grid needs as many rounds of workgroups more.  Measured, 4
+// against 8 tiles: 32/8 heads 1500 tokens 28.6 / 36.0 us, 2048 43.5 / 50.2, 3000
+// 91.0 / 81.3; 64/8 heads 1024 tokens 26.3 / 29.7, 2048 84.0 / 72.8; 16/8 heads
+// 4096 tokens 77.7 / 89.8; 32/8 heads, 1024 tokens behind 8192, 153 / 167, 1500
+// behind 1000 57.3 / 58.0, 1500 behind 8192 264 / 216.
 static bool prefill_narrow_wins(const PrefillArgs& a, int64_t blocks8, int64_t blocks4, int64_t cus) {
     if (blocks4 <= cus) return true;
     if (blocks4 > 2 * cus) return false;
@@ -1445,12 +1531,12 @@ struct Split32Plan {
 // Splits only where the 4-tile workgroups leave at least half the CUs idle and
 // the short form does not apply, and only when the estimate says it pays by a
 // tenth.  Estimates in ns, fitted to the measurements at the kernel and here:
-// unsplit 960 per key tile + 5000; split 870 per key tile of a split + 8000
+// unsplit 920 per key tile + 5000; split 870 per key tile of a split + 8000
 // (second launch, more stores) + the partials' way out and back at 3.5 TB/s.
 // 8/1 heads, 300 rows behind 1000 keys: 1 / 2 / 4 / 8 splits 23.7 / 18.3 / 15.9 /
 // 16.7 us; 32/8 heads, 7 behind 12001: 16 / 24 / 32 splits 18.3 / 17.0 / 18.1;
-// 16/8 heads, 512 behind 600: 1 / 2 splits 21.3 / 20.7; a 927-token prompt 19.0 /
-// 24.8 (paired, one split 18.5).
+// 16/8 heads, 512 behind 600: 1 / 2 splits 20.2 / 20.7; a 927-token prompt 17.8 /
+// 24.8.
 static Split32Plan split32_plan(const PrefillArgs& a, int num_kv_heads, int cus) {
     Split32Plan p = {};
     const int64_t rows = static_cast<int64_t>(a.q_len) * a.group;
@@ -1464,7 +1550,7 @@ static Split32Plan split32_plan(const PrefillArgs& a, int num_kv_heads, int cus)
     // question for kv_len <= 512.
     if (key_tiles <= 8) return p;
     const int64_t part_bytes = n_tiles * num_kv_heads * (kPrPartFloats + 64) * 4;
-    int64_t best = (960 * key_tiles + 5000) * 9 / 10;
+    int64_t best = (920 * key_tiles + 5000) * 9 / 10;
     const int64_t most = min(min(static_cast<int64_t>(kPrMaxSplits), cus / blocks), key_tiles);
     for (int64_t ns = 2; ns <= most; ++ns) {
         const int64_t t = 870 * ((key_tiles + ns - 1) / ns) + 8000 + 2 * part_bytes * ns / 3500;
