@@ -7,7 +7,8 @@
 // norm/RoPE/KV write + split-K decode + merge -> o_proj GEMV -> add +
 // post-attention RMSNorm -> gate_up GEMV with SiLU * up -> down GEMV; then the
 // final add + RMSNorm, the lm_head GEMV and the greedy argmax, which writes
-// the next token where the embedding reads it.  The last layer's attention
+// the next token where the embedding reads it.  Up to hidden 2560 each add +
+// RMSNorm inside the layers is part of the GEMV behind it (add_norm_gemv).  The last layer's attention
 // advances the device position, so consecutive replays need no host writes.
 //
 // The residual stream follows the reference's buffers: the residual add of
