@@ -251,7 +251,7 @@ def attend_prefill(q, k_cache, v_cache, out, position_start: int,
             _fail("sched_counters is smaller than grout_attn_prefill_sched_counter_bytes()")
     workspace = None
     if kv_len > 512:  # shorter key ranges never split
-        workspace = _prefill_workspace(q.device, Hq, Hkv, D, q_len, int(kv_len), int(position_start), MS)
+        workspace = _prefill_workspace(Hq, Hkv, D, q_len, int(kv_len), int(position_start), MS)
     if workspace is not None:
         _check(lib().grout_attn_prefill_ws(
             *args, None if sched_counters is None else _ptr(sched_counters), _ptr(workspace),
@@ -264,9 +264,10 @@ def attend_prefill(q, k_cache, v_cache, out, position_start: int,
     return out
 
 
-def _prefill_workspace(device, *sizes):
+def _prefill_workspace(*sizes):
     """Scratch of grout_attn_prefill_ws for these sizes from torch's allocator,
-    on the current stream; None where the call runs without: its keys are not
+    on the current device and its current stream, where the launch runs (the
+    tensors may sit on a peer device); None where the call runs without: its keys are not
     split, the stream is capturing (a graph would keep writing memory that the
     allocator has handed on), or there is no memory left."""
     nbytes = lib().grout_attn_prefill_workspace_bytes(*sizes)
@@ -276,7 +277,7 @@ def _prefill_workspace(device, *sizes):
     if torch.cuda.is_current_stream_capturing():
         return None
     try:
-        return torch.empty((nbytes,), dtype=torch.uint8, device=device)
+        return torch.empty((nbytes,), dtype=torch.uint8, device="cuda")
     except torch.cuda.OutOfMemoryError:
         return None
 
