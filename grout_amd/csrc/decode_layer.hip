@@ -397,27 +397,26 @@ __global__ __launch_bounds__(kGemvThreads) void gemv_wave_kernel(
 
 // Longer rows, up to kNormGemvMaxK = 2560, with the norm folded in (NormIn): the
 // workgroup issues the loads of the row and then of all its weights, normalises
-// the row into LDS while the weights are in flight, and each of its 8
+// the row into LDS while the weights are in flight, and each of its 8 or 12
 // wavefronts sums R rows against it (R = 2, NC = 5 chunk columns of 64 lanes).
-// The sum of squares is taken over 512 threads instead of 1024, the f16 roundings
+// The sum of squares is taken over kThreads instead of 1024, the f16 roundings
 // are those of rms_norm_decode_kernel.  Qwen3-4B token step (36 layers, position
-// 4001) 1955 -> 1882 us; 4 wavefronts 1-2% slower, 16 wavefronts 9%.  Folding
+// 4001) 1955 -> 1882 us (8 wavefronts throughout); 4 wavefronts 1-2% slower, 16 wavefronts 9%.  Folding
 // the norm into gemv_f16_kernel instead (each thread normalises its own chunks)
 // 1954-2694: every 2-row workgroup then reads 15 KB of row data for 10 KB of
 // weights.  Qwen3-32B (k = 5120) keeps its norm launches: 2125 us at best against
 // 2119 for 12 layers; a row's 10 chunk columns leave too few wavefronts
 // resident to keep HBM busy through the prologue.
 constexpr int kNormGemvMaxK = 2560;
-constexpr int kNormGemvThreads = 512;
-template <int R, bool kSilu>
-__global__ __launch_bounds__(kNormGemvThreads) void norm_gemv_kernel(const uint16_t* __restrict__ W,
-                                                                     uint16_t* __restrict__ out, NormIn in, int m,
-                                                                     int k, int half_m) {
+template <int R, bool kSilu, int kThreads>
+__global__ __launch_bounds__(kThreads) void norm_gemv_kernel(const uint16_t* __restrict__ W,
+                                                             uint16_t* __restrict__ out, NormIn in, int m, int k,
+                                                             int half_m) {
     static_assert(!kSilu || R >= 2, "a SiLU wavefront pairs R/2 gate rows with R/2 up rows");
     constexpr int kOut = kSilu ? R / 2 : R;
     constexpr int NC = kNormGemvMaxK / 8 / kWave;
-    constexpr int kWaves = kNormGemvThreads / kWave;
-    static_assert(NC * kWave <= kNormGemvThreads, "one row chunk per thread");
+    constexpr int kWaves = kThreads / kWave;
+    static_assert(NC * kWave <= kThreads, "one row chunk per thread");
     __shared__ __attribute__((aligned(16))) uint16_t s_x[NC * kWave * 8];
     __shared__ float red[kWaves];
     const int tid = threadIdx.x;
@@ -709,12 +708,28 @@ int32_t grout::add_norm_gemv(const uint16_t* residual, const uint16_t* x, const 
             hipLaunchKernelGGL((gemv_wave_kernel<2, false, true>), grid(kGemvThreads), dim3(kGemvThreads), 0, s, weight, x,
                                out, m, k, 0, in);
         }
+        return launch_status();
+    }
+    // 12 wavefronts where their workgroups are at most one per CU and those of 8
+    // are more: every CU then streams 24 rows, instead of 32 on some and 16 on
+    // the others.  k = 2560, 8 against 12 wavefronts, per launch: qkv of 6144 rows
+    // 8.0 / 7.7 us, 4608 rows 1.0-1.3 us less; 3072 gate/up pairs 0.4-0.7 us less,
+    // 2200 1.2 less.  Past one round the smaller workgroups fill in better: 7168
+    // rows 1.2-1.5 us less with 8, 4096 pairs 1.0, 9728 pairs 1.4.
+    int dev = 0, cus = 0;
+    hipError_t e = hipGetDevice(&dev);
+    if (e == hipSuccess) e = hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev);
+    if (e != hipSuccess) return static_cast<int32_t>(e);
+    constexpr int k8 = 8 * kWave, k12 = 12 * kWave;
+    const bool wide = grid(k8).x > static_cast<unsigned>(cus) && grid(k12).x <= static_cast<unsigned>(cus);
+    if (silu && wide) {
+        hipLaunchKernelGGL((norm_gemv_kernel<2, true, k12>), grid(k12), dim3(k12), 0, s, weight, out, in, m, k, m);
     } else if (silu) {
-        hipLaunchKernelGGL((norm_gemv_kernel<2, true>), grid(kNormGemvThreads), dim3(kNormGemvThreads), 0, s, weight, out,
-                           in, m, k, m);
+        hipLaunchKernelGGL((norm_gemv_kernel<2, true, k8>), grid(k8), dim3(k8), 0, s, weight, out, in, m, k, m);
+    } else if (wide) {
+        hipLaunchKernelGGL((norm_gemv_kernel<2, false, k12>), grid(k12), dim3(k12), 0, s, weight, out, in, m, k, 0);
     } else {
-        hipLaunchKernelGGL((norm_gemv_kernel<2, false>), grid(kNormGemvThreads), dim3(kNormGemvThreads), 0, s, weight, out,
-                           in, m, k, 0);
+        hipLaunchKernelGGL((norm_gemv_kernel<2, false, k8>), grid(k8), dim3(k8), 0, s, weight, out, in, m, k, 0);
     }
     return launch_status();
 }

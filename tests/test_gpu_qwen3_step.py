@@ -258,22 +258,24 @@ def test_token_step_qwen3_06b_shapes(gpu):
         runner.close()
 
 
-@pytest.mark.parametrize("hidden,inter,vocab", [
-    (8, 8, 9),          # one chunk a row; one wavefront with outputs past the end
-    (1016, 40, 515),    # one wavefront a row pair, a ragged second chunk column
-    (1024, 72, 4099),   # its longest rows; two rows a wavefront in lm_head, an odd last pair
-    (1032, 24, 100),    # rows normalised into LDS: 129 chunks of 512 threads, workgroups half empty
-    (2560, 520, 300),   # its longest rows
-    (2568, 64, 300),    # norm launches of their own
+@pytest.mark.parametrize("hidden,inter,vocab,hq,hkv", [
+    (8, 8, 9, 4, 2),          # one chunk a row; one wavefront with outputs past the end
+    (1016, 40, 515, 4, 2),    # one wavefront a row pair, a ragged second chunk column
+    (1024, 72, 4099, 4, 2),   # its longest rows; two rows a wavefront in lm_head, an odd last pair
+    (1032, 24, 100, 4, 2),    # rows normalised into LDS: 129 chunks of 512 threads, workgroups half empty
+    (2560, 520, 300, 4, 2),   # its longest rows
+    (2568, 64, 300, 4, 2),    # norm launches of their own
+    (1032, 2056, 100, 30, 5),  # 12 wavefronts: 5120 rows and 2056 pairs, both leave a part of the last workgroup
+    (2560, 3072, 300, 32, 8),  # 12 wavefronts, every workgroup full
 ])
-def test_token_step_hidden_sizes(gpu, hidden, inter, vocab):
+def test_token_step_hidden_sizes(gpu, hidden, inter, vocab, hq, hkv):
     """Two layers on both sides of the limits of the GEMV forms with the add +
     RMSNorm folded in: logits, token and caches against the oracle, the second
     step from the first one's caches."""
     import torch
     import grout_amd
 
-    m = qwen3_tiny_model(1800 + hidden, layers=2, hidden=hidden, hq=4, hkv=2, inter=inter, vocab=vocab,
+    m = qwen3_tiny_model(1800 + hidden, layers=2, hidden=hidden, hq=hq, hkv=hkv, inter=inter, vocab=vocab,
                          max_seq=64, filled=20)
     ref = copy.deepcopy(m)
     dm = _device_model(torch, m)
@@ -282,7 +284,7 @@ def test_token_step_hidden_sizes(gpu, hidden, inter, vocab):
     logits = torch.zeros((vocab,), dtype=torch.float16, device="cuda")
     print(f"[qwen3 step] hidden {hidden} inter {inter} vocab {vocab}", flush=True)
     runner = grout_amd.Qwen3DecodeRunner(
-        **dm, token=token, position=position, logits=logits, num_q_heads=4, num_kv_heads=2,
+        **dm, token=token, position=position, logits=logits, num_q_heads=hq, num_kv_heads=hkv,
         eps=m["eps"], qk_scale_f16_bits=m["qk_scale_f16_bits"], num_splits=2, block_n=32,
         prime_position=20)
     try:
