@@ -269,17 +269,27 @@ def _prefill_workspace(*sizes):
     on the current device and its current stream, where the launch runs (the
     tensors may sit on a peer device); None where the call runs without: its keys are not
     split, the stream is capturing (a graph would keep writing memory that the
-    allocator has handed on), or there is no memory left."""
-    nbytes = lib().grout_attn_prefill_workspace_bytes(*sizes)
+    allocator has handed on), or there is no memory left.
+
+    Another stream may be capturing, here or in another thread.  Memory that the
+    allocator then has to ask HIP for would be refused and end that capture, so
+    the request runs in the relaxed capture mode."""
+    L = lib()
+    nbytes = L.grout_attn_prefill_workspace_bytes(*sizes)
     if nbytes <= 0:
         return None
     torch = _torch()
     if torch.cuda.is_current_stream_capturing():
         return None
+    mode = ctypes.c_int(_lib.HIP_STREAM_CAPTURE_MODE_RELAXED)
+    exchange = L.hipThreadExchangeStreamCaptureMode
+    exchange(mode)  # leaves the thread's own mode in `mode`
     try:
-        return torch.empty((nbytes,), dtype=torch.uint8, device="cuda")
+        return torch.empty(nbytes, dtype=torch.uint8, device="cuda")
     except torch.cuda.OutOfMemoryError:
         return None
+    finally:
+        exchange(mode)
 
 
 def prefill_sched_counters(device="cuda"):

@@ -19,6 +19,8 @@ c_i64 = ctypes.c_int64
 c_vp = ctypes.c_void_p
 
 GROUT_OK = 0
+#: hipStreamCaptureModeRelaxed
+HIP_STREAM_CAPTURE_MODE_RELAXED = 2
 STATUS_NAMES = {
     0: "GROUT_OK",
     -1: "GROUT_ERR_NULL_POINTER",
@@ -153,6 +155,9 @@ def load(path: str | None = None):
         fn = getattr(lib, name)
         fn.restype = res
         fn.argtypes = args
+    # From the HIP runtime, which the library links: hipError_t (hipStreamCaptureMode*).
+    lib.hipThreadExchangeStreamCaptureMode.restype = ctypes.c_int
+    lib.hipThreadExchangeStreamCaptureMode.argtypes = [ctypes.POINTER(ctypes.c_int)]
     if path is None:
         _lib = lib
     return lib

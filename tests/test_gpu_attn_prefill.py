@@ -3,7 +3,9 @@
 Contract: |gpu - oracle| <= 2e-3 + 1e-2*|oracle| elementwise, oracle =
 benchmarks/src/bin/attention_microbench.rs:665-702 generalised to GQA on the cache.
 """
+import ctypes
 import math
+import threading
 
 import numpy as np
 import pytest
@@ -244,6 +246,88 @@ def test_key_split_workspace_and_capture(gpu):
         grout_amd.attend_prefill(q, kc, vc, torch.empty_like(q), qs)
         torch.cuda.synchronize()
         assert torch.equal(out, unsplit)
+
+
+_GLOBAL, _THREAD_LOCAL = 0, 1  # hipStreamCaptureMode
+
+
+def _capture_around(torch, stream, mode, call, own_thread):
+    """Runs `call` (in a thread of its own or here) while `stream`, a raw handle,
+    is captured; True if the graph was built and its kernel runs on replay."""
+    import grout_amd
+
+    L = grout_amd.lib()
+    flag = torch.zeros((1,), dtype=torch.int32, device="cuda")
+    torch.cuda.synchronize()
+    stream, error = ctypes.c_void_p(stream), []
+
+    def guarded():
+        try:
+            call()
+        except Exception as e:  # the capture is ended before it is raised
+            error.append(e)
+
+    assert L.hipStreamBeginCapture(stream, mode) == 0
+    if own_thread:
+        t = threading.Thread(target=guarded)
+        t.start()
+        t.join()
+    else:
+        guarded()
+    recorded = L.grout_set_position_async(flag.data_ptr(), 7, stream)
+    graph = ctypes.c_void_p()
+    ended = L.grout_graph_end(stream, ctypes.byref(graph))
+    if error:
+        raise error[0]
+    assert recorded == 0 and ended == 0, f"the capture was broken: {recorded}, {ended}"
+    assert L.grout_graph_launch(graph, stream) == 0
+    torch.cuda.synchronize()
+    L.grout_graph_destroy(graph)
+    return int(flag.item()) == 7
+
+
+@pytest.mark.parametrize("oom", [False, True])
+@pytest.mark.parametrize("mode,own_thread", [(_GLOBAL, True), (_GLOBAL, False), (_THREAD_LOCAL, False)])
+def test_key_split_scratch_leaves_other_captures_alone(gpu, mode, own_thread, oom):
+    """An eager call whose scratch the allocator does not have at hand, while
+    another stream is captured: it splits (or, with no memory left, runs unsplit)
+    and the capture goes on."""
+    import torch
+
+    import grout_amd
+
+    hq, hkv, S, qs = 32, 8, 300, 4000
+    q, kc, vc = (torch.from_numpy(a).cuda() for a in _case(651, hq, hkv, S, qs, qs + S))
+    L = grout_amd.lib()
+    nbytes = L.grout_attn_prefill_workspace_bytes(hq, hkv, D, S, qs + S, qs, qs + S)
+    assert nbytes > (4 << 20)
+    ref, out = torch.empty_like(q), torch.full_like(q, float("nan"))
+    if oom:
+        assert L.grout_attn_prefill(
+            q.data_ptr(), kc.data_ptr(), vc.data_ptr(), ref.data_ptr(), SCALE, hq, hkv, D, S, qs + S, qs, qs + S,
+            torch.cuda.current_stream().cuda_stream) == 0
+    else:
+        grout_amd.attend_prefill(q, kc, vc, ref, qs)
+    torch.cuda.synchronize()
+    captured, side = torch.cuda.Stream(), torch.cuda.Stream()
+
+    total = torch.cuda.get_device_properties(0).total_memory
+
+    def call():
+        if oom:
+            torch.cuda.set_per_process_memory_fraction((torch.cuda.memory_reserved() + (1 << 20)) / total)
+        try:
+            with torch.cuda.stream(side):
+                grout_amd.attend_prefill(q, kc, vc, out, qs)
+        finally:
+            torch.cuda.set_per_process_memory_fraction(1.0)
+
+    torch.cuda.empty_cache()
+    reserved = torch.cuda.memory_reserved()
+    print(f"[prefill scratch] capture mode {mode} own thread {own_thread} oom {oom}", flush=True)
+    assert _capture_around(torch, captured.cuda_stream, mode, call, own_thread)
+    assert oom or torch.cuda.memory_reserved() > reserved, "the allocator had the scratch at hand"
+    assert torch.equal(out, ref)
 
 
 def _short_form_applies(cus, hq, S, qs, kv_len):
