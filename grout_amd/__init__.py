@@ -279,7 +279,12 @@ def _prefill_workspace(*sizes):
     if nbytes <= 0:
         return None
     torch = _torch()
-    if torch.cuda.is_current_stream_capturing():
+    try:
+        if torch.cuda.is_current_stream_capturing():
+            return None
+    except RuntimeError:
+        # The legacy stream while a blocking stream captures: HIP refuses the
+        # question (and an allocation), but not the launch.
         return None
     mode = ctypes.c_int(_lib.HIP_STREAM_CAPTURE_MODE_RELAXED)
     exchange = L.hipThreadExchangeStreamCaptureMode

@@ -330,6 +330,38 @@ def test_key_split_scratch_leaves_other_captures_alone(gpu, mode, own_thread, oo
     assert torch.equal(out, ref)
 
 
+@pytest.mark.parametrize("mode,own_thread", [(_GLOBAL, True), (_GLOBAL, False), (_THREAD_LOCAL, False)])
+def test_key_split_on_the_legacy_stream_beside_a_blocking_capture(gpu, mode, own_thread):
+    """An eager call on the default stream while a blocking stream is captured,
+    where HIP does not say whether the default stream captures: it runs unsplit."""
+    import torch
+
+    import grout_amd
+
+    hq, hkv, S, qs = 32, 8, 5, 4000
+    q, kc, vc = (torch.from_numpy(a).cuda() for a in _case(652, hq, hkv, S, qs, qs + S))
+    L = grout_amd.lib()
+    assert L.grout_attn_prefill_workspace_bytes(hq, hkv, D, S, qs + S, qs, qs + S) > 0
+    ref, out = torch.empty_like(q), torch.full_like(q, float("nan"))
+    legacy = torch.cuda.default_stream()
+    assert L.grout_attn_prefill(
+        q.data_ptr(), kc.data_ptr(), vc.data_ptr(), ref.data_ptr(), SCALE, hq, hkv, D, S, qs + S, qs, qs + S,
+        legacy.cuda_stream) == 0
+
+    def call():
+        with torch.cuda.stream(legacy):
+            grout_amd.attend_prefill(q, kc, vc, out, qs)
+
+    blocking = ctypes.c_void_p()
+    assert L.hipStreamCreate(ctypes.byref(blocking)) == 0
+    print(f"[prefill legacy stream] capture mode {mode} own thread {own_thread}", flush=True)
+    try:
+        assert _capture_around(torch, blocking.value, mode, call, own_thread)
+    finally:
+        assert L.hipStreamDestroy(blocking) == 0
+    assert torch.equal(out, ref)
+
+
 def _short_form_applies(cus, hq, S, qs, kv_len):
     """The host rule of the short form: every 32-row block needs at most 8 key
     tiles of 64, and one workgroup per (query head, row block) fits the CUs."""
