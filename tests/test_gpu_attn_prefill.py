@@ -119,19 +119,17 @@ def test_prefill_long_sampled_rows(gpu, S):
 
 @pytest.mark.parametrize("S,G,qs", [(1024, 4, 0), (700, 2, 300)])
 def test_small_grid_workgroup_shape_is_bit_identical(gpu, S, G, qs):
-    """Grids that fill at most half the CUs run 4-wavefront workgroups, larger
-    ones 8-wavefront workgroups; every wavefront computes the same thing in
+    """Grids of at most one 4-tile workgroup per CU run those, grids of more than
+    two per CU 8-tile workgroups; every wavefront computes the same thing in
     both, so a problem and the same problem with more KV heads appended (which
     pushes the grid past the threshold) agree bit for bit on the shared heads."""
     import torch
 
     cus = torch.cuda.get_device_properties(0).multi_processor_count
-    n_pos = -(-S // 32)
-    hkv_small = 2
-    while 2 * (-(-n_pos * G // 8)) * (hkv_small + 1) <= cus:
-        hkv_small += 1
-    hkv_big = 2 * hkv_small
-    assert 2 * (-(-n_pos * G // 8)) * hkv_small <= cus < 2 * (-(-n_pos * G // 8)) * hkv_big
+    per_head = -(-(-(-S // 32) * G) // 4)  # 4-tile workgroups
+    hkv_small = cus // per_head
+    hkv_big = 2 * cus // per_head + 1
+    assert hkv_small >= 2 and per_head * hkv_small <= cus and per_head * hkv_big > 2 * cus
     print(f"[prefill 4/8 waves] S={S} G={G} Hkv {hkv_small} vs {hkv_big}", flush=True)
     q, kc, vc = _case(400 + S, hkv_big * G, hkv_big, S, qs, qs + S)
     small = _run(torch, np.ascontiguousarray(q[:, :hkv_small * G]), np.ascontiguousarray(kc[:hkv_small]),
@@ -148,7 +146,8 @@ def test_small_grid_workgroup_shape_is_bit_identical(gpu, S, G, qs):
     (1000, 4, 8, 0),    # one round of 4-tile workgroups, ragged last tile
     (1024, 8, 8, 0),    # two rounds: 512 workgroups on 256 CUs
     (33, 3, 2, 700),    # a handful of workgroups, tasks past the end, 12 tiles
-    (65, 1, 5, 0),      # shortest walks: 1 and 2 tiles
+    (65, 1, 5, 0),      # behind 520 keys: walks of 9 and 10 tiles
+    (65, 1, 90, 0),     # shortest walks, 1 and 2 tiles: too many heads for the short form
 ])
 def test_narrow_workgroups_are_bit_identical(gpu, S, G, hkv, qs):
     """4-tile workgroups (computing and copying wavefronts apart) against the
@@ -161,7 +160,7 @@ def test_narrow_workgroups_are_bit_identical(gpu, S, G, hkv, qs):
     hkv_big = hkv * (-(-4 * cus // (-(-n_pos * G // 8) * hkv)))
     print(f"[prefill narrow] S={S} G={G} Hkv {hkv} vs {hkv_big}", flush=True)
     # Past the short form's 8 key tiles, or past its one workgroup per CU.
-    kv_pad = 520 if qs + S <= 512 else 0
+    kv_pad = 520 if _short_form_applies(cus, hkv * G, S, qs, qs + S) else 0
     g = torch.Generator(device="cuda").manual_seed(500 + S)
     q, kc, vc = (torch.randn(s, generator=g, device="cuda", dtype=torch.float16)
                  for s in ((S, hkv_big * G, D), (hkv_big, qs + S + kv_pad, D), (hkv_big, qs + S + kv_pad, D)))
@@ -246,6 +245,65 @@ def test_key_split_workspace_and_capture(gpu):
         grout_amd.attend_prefill(q, kc, vc, torch.empty_like(q), qs)
         torch.cuda.synchronize()
         assert torch.equal(out, unsplit)
+
+
+@pytest.mark.parametrize("hq,hkv,S", [
+    (1, 1, 4000),  # 32 workgroups, the lightest with one row tile
+    (2, 1, 2000),  # two query heads packed
+])
+def test_key_split_with_empty_splits(gpu, hq, hkv, S):
+    """A prompt from position 0 whose first row blocks have fewer key tiles than
+    there are splits: workgroups without a tile leave partials of weight 0, and
+    every partial that the merge reads has been written (the workspace is NaN)."""
+    import torch
+
+    import grout_amd
+
+    L = grout_amd.lib()
+    nbytes = L.grout_attn_prefill_workspace_bytes(hq, hkv, D, S, S, 0, S)
+    n_tiles = -(-S * (hq // hkv) // 32)
+    splits = nbytes // (32 * (D + 2) * 4 * hkv * n_tiles)
+    # Workgroups take 4 row tiles, heaviest first: the lightest has the remainder.
+    lightest_rows = 32 * ((n_tiles - 1) % 4 + 1)
+    assert splits > -(-(lightest_rows // (hq // hkv)) // 64), "no split is empty"
+    print(f"[prefill empty splits] hq={hq} hkv={hkv} S={S} splits {splits}", flush=True)
+    h = _case(670 + hq, hq, hkv, S, 0, S, scale_rows=0.01)
+    q, kc, vc = (torch.from_numpy(a).cuda() for a in h)
+    out = torch.full_like(q, float("nan"))
+    ws = torch.full((nbytes // 4,), float("nan"), device="cuda")
+    assert L.grout_attn_prefill_ws(
+        q.data_ptr(), kc.data_ptr(), vc.data_ptr(), out.data_ptr(), SCALE, hq, hkv, D, S, S, 0, S, None,
+        ws.data_ptr(), nbytes, torch.cuda.current_stream().cuda_stream) == 0
+    torch.cuda.synchronize()
+    ref = oracle.attn_prefill_f32(*h, SCALE, kv_len=S, query_start=0)
+    assert_close_attn(out.cpu().numpy(), ref, f"empty splits hq={hq} S={S}")
+
+
+def test_key_split_on_two_streams(gpu):
+    """Split launches of two problems on two streams at once: each takes scratch
+    of its own stream, so both give what they give alone."""
+    import torch
+
+    import grout_amd
+
+    hq, hkv = 32, 8
+    problems = []
+    for i, (S, qs) in enumerate(((7, 9000), (61, 5000))):
+        q, kc, vc = (torch.from_numpy(a).cuda() for a in _case(680 + i, hq, hkv, S, qs, qs + S))
+        assert grout_amd.lib().grout_attn_prefill_workspace_bytes(hq, hkv, D, S, qs + S, qs, qs + S) > 0
+        ref = torch.empty_like(q)
+        grout_amd.attend_prefill(q, kc, vc, ref, qs)
+        outs = [torch.full_like(q, float("nan")) for _ in range(40)]
+        problems.append((torch.cuda.Stream(), q, kc, vc, ref, outs, qs))
+    torch.cuda.synchronize()
+    print("[prefill key split] two streams", flush=True)
+    for i in range(40):
+        for stream, q, kc, vc, _, outs, qs in problems:
+            with torch.cuda.stream(stream):
+                grout_amd.attend_prefill(q, kc, vc, outs[i], qs)
+    torch.cuda.synchronize()
+    for _, _, _, _, ref, outs, _ in problems:
+        assert all(torch.equal(o, ref) for o in outs)
 
 
 _GLOBAL, _THREAD_LOCAL = 0, 1  # hipStreamCaptureMode
