@@ -171,10 +171,11 @@ def test_decode_equals_prefill_row(gpu):
 
 @pytest.mark.parametrize("scale,start", [
     (1.0, 0), (1.0, 40000),   # angles up to 4e4 and below 1e-2
-    (3.0e4, 35700),           # past 2^30: the large-angle path for some frequencies
-    (1.0e25, 35700),          # all of them
+    (3.0e4, 35700),           # up to 0.998 of 2^30
+    (4.0e4, 35700),           # past 2^30 for two frequencies: a wavefront takes both paths
+    (1.0e25, 35700),          # the large-angle path alone
 ])
-def test_angles_correctly_rounded(gpu, scale, start):
+def test_angles_within_f16_rounding(gpu, scale, start):
     """cos and sin of the f32 angles, read back through the op: a row of ones
     under weight ones gives cos - sin and cos + sin of each frequency, here held
     to float64 within f16 rounding (half an ulp, plus the f32 roundings of the two
@@ -193,7 +194,48 @@ def test_angles_correctly_rounded(gpu, scale, start):
     got = out[:, 0].double().cpu()
     pos = torch.arange(start, start + S, dtype=torch.float32)
     theta = (pos[:, None] * inv[None, :]).numpy().astype(np.float64)
+    past = (theta >= 2.0 ** 30).any(0)
+    assert past.any() == (scale >= 4.0e4) and past.all() == (scale == 1.0e25)
     c, s = torch.from_numpy(np.cos(theta)), torch.from_numpy(np.sin(theta))
     ref = torch.cat([c - s, c + s], dim=1)
     ulp = torch.clamp(2.0 ** (torch.floor(torch.log2(ref.abs().clamp_min(2.0 ** -14))) - 10), min=2.0 ** -24)
     assert bool(((got - ref).abs() <= 0.5 * ulp + 1.5 * 2.0 ** -23).all())
+
+
+@pytest.mark.parametrize("scale,last", [(1.0, 40000), (3.0e4, 35790), (4.0e4, 40000), (1.0e25, 40000)])
+def test_angles_correctly_rounded(gpu, scale, last):
+    """cos and sin of the f32 angles to the last f32 bit, through the f16 output:
+    the weights of frequency j are an f16 pair (a, b) next to (sin, cos) * K, so
+    that a * cos - b * sin cancels to ~K * 2^-20 and its f16 value shows f32
+    roundings of both products.  The op's f32 steps (x = 1, inverse RMS 1, no
+    contraction) on the f32 values nearest to the f64 cos and sin give the
+    expected bits; an angle's f64 error of 1e-16 moves such an f32 value once in
+    10^8."""
+    import torch
+    import grout_amd
+
+    inv = grout_amd.build_inv_freq(1e6) * scale
+    g = rng(1900)
+    positions = np.unique(np.concatenate([[0, 1, last], g.integers(0, last + 1, 29)]))
+    theta = (positions.astype(np.float32)[:, None] * inv.numpy()[None, :]).astype(np.float64)
+    assert (theta >= 2.0 ** 30).any() == (scale >= 4.0e4)
+    c, s = np.cos(theta), np.sin(theta)
+    k = np.arange(1024.0, 2048.0)[:, None, None]
+    a, b = (k * s).astype(np.float16), (k * c).astype(np.float16)
+    best = np.abs(a.astype(np.float64) * c - b.astype(np.float64) * s).argmin(0)[None]
+    a, b = np.take_along_axis(a, best, 0)[0], np.take_along_axis(b, best, 0)[0]
+    c32, s32, a32, b32 = (t.astype(np.float32) for t in (c, s, a, b))
+    expect = np.concatenate([a32 * c32 - b32 * s32, b32 * c32 + a32 * s32], 1).astype(np.float16)
+    # The pairs do show f32 roundings: one ulp more on cos changes most of them.
+    c_up = np.nextafter(c32, np.float32(2))
+    seen = (a32 * c_up - b32 * s32).astype(np.float16) != expect[:, :64]
+    assert seen[(c != 0) & (s != 0) & (theta > 0.1)].mean() > 0.5
+    ones = torch.ones((1, 1, 128), dtype=torch.float16, device="cuda")
+    out = torch.empty((len(positions), 1, 128), dtype=torch.float16, device="cuda")
+    cache = torch.zeros((1, last + 1, 128), dtype=torch.float16, device="cuda")
+    w = torch.from_numpy(np.concatenate([a, b], 1)).cuda()
+    print(f"[rope angles] scale {scale} positions to {last}", flush=True)
+    for i, p in enumerate(positions):
+        grout_amd.qk_norm_rope_kv_prefill(ones, ones, ones, w[i], w[i], inv.cuda(), out[i:i + 1], cache, cache, 0.0,
+                                          int(p))
+    assert np.array_equal(out[:, 0].cpu().numpy().view(np.uint16), expect.view(np.uint16))
