@@ -15,6 +15,7 @@ Contract:
   issued back to back from C agree to the same tolerance.
 """
 import copy
+import ctypes
 
 import numpy as np
 import pytest
@@ -95,6 +96,95 @@ def test_gemv_silu_mul_equals_two_launches(gpu, n, k, seed):
     grout_amd.gemv_silu_mul(dw, dx, out)
     torch.cuda.synchronize()
     assert torch.equal(out.view(torch.int16), ref[:n].view(torch.int16))
+
+
+def _add_norm_gemv(torch, residual, x, norm_weight, eps, weight, silu):
+    """grout::add_norm_gemv (csrc/decode_layer.h), which has no C entry point: the
+    token step's add + RMSNorm and the GEMV behind it in one launch."""
+    import grout_amd
+
+    f = grout_amd.lib()._ZN5grout13add_norm_gemvEPKtS1_S1_PtfS1_S2_iibP12ihipStream_t
+    f.restype = ctypes.c_int32
+    p = ctypes.c_void_p
+    f.argtypes = [p] * 4 + [ctypes.c_float, p, p, ctypes.c_int32, ctypes.c_int32, ctypes.c_bool, p]
+    m, k = weight.shape
+    m = m // 2 if silu else m
+    out = torch.full((m,), float("nan"), dtype=torch.float16, device="cuda")
+    res = torch.full((k,), float("nan"), dtype=torch.float16, device="cuda")
+    st = f(residual.data_ptr(), x.data_ptr(), norm_weight.data_ptr(), res.data_ptr(), eps, weight.data_ptr(),
+           out.data_ptr(), m, k, silu, torch.cuda.current_stream().cuda_stream)
+    assert st == 0, f"status {st}"
+    return out, res
+
+
+@pytest.mark.parametrize("n,k", [
+    (1, 8),         # two rows, one chunk
+    (5, 24),        # wavefronts past the end
+    (37, 520),      # one wavefront a row pair, a second chunk column of one chunk
+    (333, 1016),    # a ragged one
+    (2050, 1024),   # its longest rows
+    (7, 1032),      # rows normalised into LDS: 129 chunks of 512 threads
+    (2056, 1032),   # 12 wavefronts, a part of the last workgroup
+    (4101, 2048),   # 8 wavefronts in several rounds
+    (520, 2560),    # the longest rows
+    (3072, 2560),   # 12 wavefronts, every workgroup full
+])
+def test_folded_norm_gemv_equals_its_launches(gpu, n, k):
+    """The GEMVs with the add + RMSNorm folded in against the launches they stand
+    for, on 2n rows; the SiLU form on n gate/up pairs equals SiLU * up of the
+    plain form's rows bit for bit, and the residual output the norm launch's.
+
+    Bound of a row sum, A = sum |w n| over its normalised inputs n in f64: both
+    sides sum f32 products in chains of at most 64 roundings (dot products, lane
+    and wavefront sums, sum of squares, inverse RMS) of 2^-24 each, then round
+    to f16.  Rows of more than 1024 take n in f16 as the launches do, but the
+    inverse RMS may differ by 64 * 2^-24 and move the n closer than that to an f16
+    midpoint by an ulp.  Shorter rows do not round n to f16, which the launches
+    do: they are held to f64."""
+    import torch
+    import grout_amd
+
+    g = rng(1850 + n)
+    eps = 1e-6
+    residual, x = normal_f16(g, k), normal_f16(g, k, 0.5)
+    nw = (1.0 + 0.1 * g.standard_normal(k)).astype(np.float16)
+    w = normal_f16(g, (2 * n, k), 1.0 / np.sqrt(k))
+    dres, dx, dnw, dw = (_dev(torch, a) for a in (residual, x, nw, w))
+    print(f"[folded norm] n={n} k={k}", flush=True)
+    rows, res = _add_norm_gemv(torch, dres, dx, dnw, eps, dw, False)
+    ff, res_silu = _add_norm_gemv(torch, dres, dx, dnw, eps, dw, True)
+    normed, res_ref = torch.empty_like(dx), torch.empty_like(dx)
+    grout_amd.add_rms_norm_decode(dres, dx, dnw, normed, res_ref, eps)
+    rows_ref = torch.empty_like(rows)
+    grout_amd.gemv_f16(dw, normed, rows_ref)
+    n8 = -(-n // 8) * 8  # silu_mul takes whole 16-byte chunks
+    gate, up, ff_ref = (torch.zeros((n8,), dtype=torch.float16, device="cuda") for _ in range(3))
+    gate[:n], up[:n] = rows[:n], rows[n:]
+    grout_amd.silu_mul(gate, up, ff_ref)
+    torch.cuda.synchronize()
+    assert torch.equal(res.view(torch.int16), res_ref.view(torch.int16))
+    assert torch.equal(res_silu.view(torch.int16), res_ref.view(torch.int16))
+    assert torch.equal(ff.view(torch.int16), ff_ref[:n].view(torch.int16))
+
+    c = residual.astype(np.float64) + x.astype(np.float64)
+    n64 = c / np.sqrt(np.mean(c * c) + eps) * nw.astype(np.float64)
+    w64 = w.astype(np.float64)
+    chain = 64 * 2.0 ** -24
+    sums = np.abs(w64) @ np.abs(n64)
+    got = rows.cpu().numpy()
+    if k <= 1024:
+        ref = w64 @ n64
+        bound = chain * sums
+    else:
+        ref = rows_ref.cpu().numpy().astype(np.float64)
+        ulp = np.spacing(np.abs(n64).astype(np.float16)).astype(np.float64)
+        frac = np.abs(n64) / ulp % 1.0
+        near = np.abs(frac - 0.5) * ulp <= chain * np.abs(n64)
+        bound = 2 * chain * sums + np.abs(w64) @ np.where(near, ulp, 0.0)
+    # Each side rounds its sum to f16: half an ulp of the larger value.
+    half = 0.5 * np.spacing((np.abs(ref) + bound).astype(np.float16)).astype(np.float64)
+    err = np.abs(got.astype(np.float64) - ref)
+    assert (err <= bound + (1 if k <= 1024 else 2) * half).all(), (err - bound).max()
 
 
 def _device_model(torch, m):
