@@ -494,3 +494,58 @@ def test_python_mirror_shape_errors():
     with pytest.raises(grout_amd.GroutError, match="weight must have 64 elements"):
         z = torch.zeros(64, dtype=h)
         grout_amd.add_rms_norm_decode(z, z, torch.zeros(32, dtype=h), z, z, 1e-6)
+
+
+@pytest.mark.parametrize("capturing", [False, True, RuntimeError])
+@pytest.mark.parametrize("nbytes,memory", [(4096, True), (4096, False), (0, True), (-6, True)])
+def test_prefill_scratch_of_the_wrapper(monkeypatch, capturing, nbytes, memory):
+    """attend_prefill's scratch is asked for on the current device, where the
+    launch runs (never a tensor's own device), in the relaxed capture mode, and
+    the thread's mode is put back; without a split, under capture or without
+    memory there is none."""
+    import grout_amd
+
+    class OutOfMemory(RuntimeError):
+        pass
+
+    asked, modes = [], []
+
+    class Torch:
+        uint8 = "uint8"
+
+        class cuda:
+            OutOfMemoryError = OutOfMemory
+
+            @staticmethod
+            def is_current_stream_capturing():
+                if capturing is RuntimeError:
+                    raise RuntimeError("the legacy stream beside a blocking stream's capture")
+                return capturing
+
+        @staticmethod
+        def empty(n, dtype, device):
+            asked.append((n, dtype, device, modes[-1]))
+            if not memory:
+                raise OutOfMemory
+            return "scratch"
+
+    class Lib:
+        mode = 1  # the thread's own: thread-local
+
+        @staticmethod
+        def grout_attn_prefill_workspace_bytes(*sizes):
+            return nbytes
+
+        @classmethod
+        def hipThreadExchangeStreamCaptureMode(cls, mode):
+            cls.mode, mode.value = mode.value, cls.mode
+            modes.append(cls.mode)
+            return 0
+
+    monkeypatch.setattr(grout_amd, "lib", lambda: Lib)
+    monkeypatch.setattr(grout_amd, "_torch", lambda: Torch)
+    got = grout_amd._prefill_workspace(32, 8, 128, 7, 4007, 4000, 4096)
+    eager = nbytes > 0 and capturing is False
+    assert got == ("scratch" if eager and memory else None)
+    assert asked == ([(nbytes, "uint8", "cuda", 2)] if eager else [])
+    assert Lib.mode == 1
