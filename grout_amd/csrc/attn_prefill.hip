@@ -649,10 +649,10 @@ __global__ __launch_bounds__(kPfWaves * kWave, 1) void attn_prefill_kernel(Prefi
     half8_t pop[4];  // P^T of the last softmaxed tile
 #pragma unroll
     for (int k = 0; k < 4; ++k) pop[k] = half8_t{};
-    // The V half of the last stage is what GEMM(0) multiplies with P = 0:
-    // zero it (finite), before the first barrier.  Tile 3 refills it only
-    // after both groups are past GEMM(0).
-    {
+    // The V half of the last stage is what GEMM(0) of the 8-wavefront forms
+    // multiplies with P = 0: zero it (finite), before the first barrier.  Tile 3
+    // refills it only after both groups are past GEMM(0).
+    if constexpr (kWaves != 4) {
         uint4_t* vz = reinterpret_cast<uint4_t*>(pf_lds + (kPfStages - 1) * kPfStageBytes + kPfKBytes);
         for (int i = tid; i < kPfVBytes / 16; i += kWaves * kWave) vz[i] = uint4_t{0u, 0u, 0u, 0u};
     }
@@ -665,11 +665,11 @@ __global__ __launch_bounds__(kPfWaves * kWave, 1) void attn_prefill_kernel(Prefi
     const uint32_t k_lane = (l32 & 15) * kPfKBlock + (l32 >> 4) * 256 + 16 * hl;
     const uint32_t v_lane = (4 * (gi >> 1) + (ii >> 2)) * kPfVBlock + 32 * (gi & 1) + 8 * (ii & 3);
 
-    // GEMM phase of tile j: PV of tile j-1, then S of tile j.
+    // GEMM phase of tile j (8-wavefront forms): PV of tile j-1, then S of tile j.
     //
     // Every GEMM phase runs all 32 slots (one code path keeps register
     // allocation tight): at j = 0 the PV half multiplies P = 0 with the V
-    // stage zeroed below (adds exactly +0 to O); at j = wave_tiles the S half
+    // stage zeroed above (adds exactly +0 to O); at j = wave_tiles the S half
     // reads a stage inside LDS and its result is never used.
     // A split wavefront whose range starts after the workgroup's first tile
     // runs the GEMM phases before it too: its P is still zero there (PV adds
@@ -713,15 +713,15 @@ __global__ __launch_bounds__(kPfWaves * kWave, 1) void attn_prefill_kernel(Prefi
         pf_softmax<2>(s, pop, o, m_run, l_run, c);
     };
 
-    // Tile step t: group A runs GEMM(t) then softmax(t), group B softmax(t-1)
-    // then GEMM(t).  GEMM(ntiles) is the last PV; softmax of a tile outside
-    // the wavefront's range is a no-op.  Each group has its own straight-line
-    // loop (B's is A's rotated by one phase); both pass the same ntiles+1
-    // barriers, one at the start of each step.  Tile t+2 is issued after the
-    // barrier of step t into the stage of tile t-2, whose last reader (group
+    // 8-wavefront forms, tile step t: group A runs GEMM(t) then softmax(t), group
+    // B softmax(t-1) then GEMM(t).  GEMM(ntiles) is the last PV; softmax of a tile
+    // outside the wavefront's range is a no-op.  Each group has its own
+    // straight-line loop (B's is A's rotated by one phase); both pass the same
+    // ntiles+1 barriers, one at the start of each step.  Tile t+2 is issued after
+    // the barrier of step t into the stage of tile t-2, whose last reader (group
     // B's GEMM(t-1), the PV of tile t-2) ended before that barrier.
     auto open_tile_step = [&](int t) {
-        if constexpr (kWaves != 4) wait_tile(t);
+        wait_tile(t);
         pf_barrier();
     };
     // The copies of tile t+2 go out at the start of each wavefront's softmax
