@@ -1102,11 +1102,12 @@ __global__ __launch_bounds__(kSpWaves * kWave, 1) void attn_prefill_short_kernel
 //    after the barrier of step t, into the slots that GEMM(t-1) read last, three
 //    steps before GEMM(t+2) and GEMM(t+3) need them.
 // Bound by the copies with one or two row tiles per KV head (a CU takes ~40
-// bytes a cycle into LDS, HBM gives each ~28), by the phases' fixed latencies
-// (~2000 cycles a 64-key step) with more.  Measured, unsplit -> split kernel and
-// merge: 32/8 heads, 7 rows behind 12001 keys 166 -> 17.0 us (2.9 TB/s of K/V),
-// 509 behind 6003 95 -> 65; 64/8 heads, 10 behind 28683 389 -> 34 (3.5 TB/s);
-// 16/8 heads, 5 behind 3000 45 -> 10.8.
+// bytes a cycle into LDS, HBM gives each ~28 GB/s, 12 bytes a cycle), by the
+// phases' fixed latencies (~2000 cycles a 64-key step) with more.  Measured,
+// the 4-tile grid above -> split kernel and merge: 32/8 heads, 7 rows behind
+// 12001 keys 156 -> 18.7 us (2.6 TB/s of K/V), 509 behind 6003 90 -> 67; 64/8
+// heads, 10 behind 28683 366 -> 30.8 (3.8 TB/s); 16/8 heads, 5 behind 3000 42.5
+// -> 10.5.
 constexpr int kPrWaves = 8;      // computing wavefronts
 constexpr int kPrCopyWaves = 4;  // and copying ones
 constexpr int kPrThreads = (kPrWaves + kPrCopyWaves) * kWave;
@@ -1452,13 +1453,15 @@ static int64_t prefill_rounds(int64_t blocks, int64_t cus, int64_t most, int64_t
     return t;
 }
 
-// Whether 4-tile workgroups (blocks4) beat 8-tile ones (blocks8).  A step of
-// the former takes about 4/5 of a step of the latter (0.92 against 1.22 us), so
-// they lose once the grid needs as many rounds of workgroups more.  Measured, 4
-// against 8 tiles: 32/8 heads 1500 tokens 28.6 / 36.0 us, 2048 43.5 / 50.2, 3000
-// 91.0 / 81.3; 64/8 heads 1024 tokens 26.3 / 29.7, 2048 84.0 / 72.8; 16/8 heads
-// 4096 tokens 77.7 / 89.8; 32/8 heads, 1024 tokens behind 8192, 153 / 167, 1500
-// behind 1000 57.3 / 58.0, 1500 behind 8192 264 / 216.
+// Whether 4-tile workgroups (blocks4) beat 8-tile ones (blocks8).  In steps of
+// prefill_rounds the launches below took 0.92-1.15 us a step with the former,
+// 1.22-1.50 with the latter, 0.67 to 0.82 of it at one shape.  The rule counts
+// 4/5: the former lose once the grid needs that many more rounds.  Measured, 4
+// against 8 tiles: 32/8 heads 1500 tokens 30.4 / 37.4 us, 2048 46.9 / 50.5, 3000
+// 91.2 / 81.1; 64/8 heads 1024 tokens 26.9 / 29.9, 1500 52.3 / 45.8, 2048 82.9 /
+// 72.5; 16/8 heads 3000 tokens 49.2 / 61.5, 4096 77.2 / 89.2; 32/8 heads, 1024
+// tokens behind 8192, 149 / 168, 1100 behind 1000 44.5 / 45.2, 1500 behind 8192
+// 259 / 214.  1500 behind 1000, 56.4 / 57.6, goes to 8 tiles.
 static bool prefill_narrow_wins(const PrefillArgs& a, int64_t blocks8, int64_t blocks4, int64_t cus) {
     if (blocks4 <= cus) return true;
     if (blocks4 > 2 * cus) return false;
@@ -1529,14 +1532,17 @@ struct Split32Plan {
 };
 
 // Splits only where the 4-tile workgroups leave at least half the CUs idle and
-// the short form does not apply, and only when the estimate says it pays by a
-// tenth.  Estimates in ns, fitted to the measurements at the kernel and here:
-// unsplit 920 per key tile + 5000; split 870 per key tile of a split + 8000
-// (second launch, more stores) + the partials' way out and back at 3.5 TB/s.
+// the short form does not apply, and only when the estimate says it pays.
+// Estimates in ns, fitted to the measurements at the kernel and here: unsplit
+// 828 per key tile + 4500; split 870 per key tile of a split + 8000 (second
+// launch, more stores) + the partials' way out and back at 3.5 TB/s.  Measured
+// at the fewest key tiles that split, unsplit / split: 32/8 heads, 5 rows and 9
+// tiles 11.9 / 8.8 us, 33 and 9 12.6 / 12.9, 130 and 15 18.0 / 16.8, 512 and 36
+// 35.1 / 35.4; 64/8 heads, 33 and 12 15.2 / 14.4; 16/8 heads, 64 and 9 12.6 /
+// 13.1, 512 and 21 22.6 / 21.9; 8/1 heads, 130 and 9 12.7 / 13.1; at five more
+// tiles the split takes 0.59-0.97 of the unsplit time in each.  Split counts:
 // 8/1 heads, 300 rows behind 1000 keys: 1 / 2 / 4 / 8 splits 23.7 / 18.3 / 15.9 /
-// 16.7 us; 32/8 heads, 7 behind 12001: 16 / 24 / 32 splits 18.3 / 17.0 / 18.1;
-// 16/8 heads, 512 behind 600: 1 / 2 splits 20.2 / 20.7; a 927-token prompt 17.8 /
-// 24.8.
+// 16.7 us; 32/8 heads, 7 behind 12001: 16 / 24 / 32 splits 18.3 / 17.0 / 18.1.
 static Split32Plan split32_plan(const PrefillArgs& a, int num_kv_heads, int cus) {
     Split32Plan p = {};
     const int64_t rows = static_cast<int64_t>(a.q_len) * a.group;
@@ -1550,7 +1556,7 @@ static Split32Plan split32_plan(const PrefillArgs& a, int num_kv_heads, int cus)
     // question for kv_len <= 512.
     if (key_tiles <= 8) return p;
     const int64_t part_bytes = n_tiles * num_kv_heads * (kPrPartFloats + 64) * 4;
-    int64_t best = (920 * key_tiles + 5000) * 9 / 10;
+    int64_t best = 828 * key_tiles + 4500;
     const int64_t most = min(min(static_cast<int64_t>(kPrMaxSplits), cus / blocks), key_tiles);
     for (int64_t ns = 2; ns <= most; ++ns) {
         const int64_t t = 870 * ((key_tiles + ns - 1) / ns) + 8000 + 2 * part_bytes * ns / 3500;
