@@ -101,9 +101,9 @@ template <int n>
 constexpr double kInvFact = inv_factorial_of(n);
 
 // sin and cos of an f32 angle, each rounded once to f32 from an f64 value good
-// to ~1e-16.  theta = n pi/2 + r with |r| <= pi/4: pi/2's f64 value is a multiple
-// of 2^-52, so x - n hi is exact in one FMA, and the second FMA takes n times the
-// rest of pi/2.  Taylor series in r^2 to r^17 and r^16 (the terms left out are
+// to ~1e-16.  Cody and Waite's two-term reduction, theta = n pi/2 + r with |r| <=
+// pi/4: pi/2's f64 value is a multiple of 2^-52, so x - n hi is exact in one FMA,
+// and the second FMA takes n times the rest of pi/2.  Taylor series in r^2 to r^17 and r^16 (the terms left out are
 // below 2e-18), summed pairwise: a launch waits for one such chain, and the
 // library's sincos is ~1600 cycles long.  Angles of 2^30 and more, infinities and
 // NaN take the library's.

@@ -321,8 +321,9 @@ struct NormIn {
 // its rows and of x; the sums need six shuffles and no LDS.  gemv_f16_kernel
 // spreads a row over 256 threads, half of which have no chunk at k = 1024.
 // Measured, there -> here: 4096 rows 3.49 -> 3.33 us, 3072 gate/up pairs 4.47 ->
-// 4.17, 151936 rows 52 -> 47.3 us (5.9 -> 6.6 TB/s); longer rows lose (k 2048
-// 2.85 -> 3.35 us, k 2560 16.5 -> 17.6).
+// 4.17, 151936 rows 52 -> 47.3 us (5.9 -> 6.6 TB/s); shorter rows gain more
+// (151936 rows of 64 38.5 -> 15.1 us) and no count from 1 row up loses (1 row of
+// 64 1.95 -> 1.93); longer rows lose (k 2048 2.85 -> 3.35 us, k 2560 16.5 -> 17.6).
 // kNorm: x is the RMSNorm of in.residual + in.x (see NormIn).  Each wavefront
 // takes the row sums on c * w, c = residual + x in f32, sums c^2 beside them and
 // scales at the end: W (c * inv * w) = inv * (W (c * w)), so nothing waits for
@@ -400,12 +401,17 @@ __global__ __launch_bounds__(kGemvThreads) void gemv_wave_kernel(
 // the row into LDS while the weights are in flight, and each of its 8 or 12
 // wavefronts sums R rows against it (R = 2, NC = 5 chunk columns of 64 lanes).
 // The sum of squares is taken over kThreads instead of 1024, the f16 roundings
-// are those of rms_norm_decode_kernel.  Qwen3-4B token step (36 layers, position
-// 4001) 1955 -> 1882 us (8 wavefronts throughout); 4 wavefronts 1-2% slower, 16 wavefronts 9%.  Folding
-// the norm into gemv_f16_kernel instead (each thread normalises its own chunks)
-// 1954-2694: every 2-row workgroup then reads 15 KB of row data for 10 KB of
-// weights.  Qwen3-32B (k = 5120) keeps its norm launches: 2125 us at best against
-// 2119 for 12 layers; a row's 10 chunk columns leave too few wavefronts
+// are those of rms_norm_decode_kernel.  Token steps, norm launches -> folded:
+// Qwen3-4B (36 layers, position 4001) 1928 -> 1847 us; 12 layers of hidden 1032
+// 331 -> 291, 1536 447 -> 418, 2048 448 -> 414, 2304 520 -> 495.  4 wavefronts
+// throughout are 1-2% slower than 8, 16 wavefronts 9%.  Folding the norm into
+// gemv_f16_kernel instead (each thread normalises its own chunks) took 1954-2694
+// us a Qwen3-4B step when the launches took 1955: every 2-row workgroup then
+// reads 15 KB of row data for 10 KB of weights.  The limit is the kernel's chunk
+// columns: with NC = 8 (k to 4096) hidden 2560 loses 2% (12 layers 584 -> 597 us,
+// 64 weight registers a thread instead of 40), while 2568 and 3072 would gain 4%
+// and 5% over their norm launches, 4096 1%.  With 10 columns Qwen3-32B (k = 5120)
+// takes 2125 us at best against 2119 for 12 layers: too few wavefronts stay
 // resident to keep HBM busy through the prologue.
 constexpr int kNormGemvMaxK = 2560;
 template <int R, bool kSilu, int kThreads>
