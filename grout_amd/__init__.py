@@ -228,8 +228,12 @@ def attend_prefill(q, k_cache, v_cache, out, position_start: int,
     f32 (:5601).  With `sched_counters` (prefill_sched_counters()) the launch
     uses the dynamic per-XCD schedule (grout_attn_prefill_sched); the result
     is bit-identical to the static grid's.  A few rows behind many keys take
-    grout_attn_prefill_ws with scratch from torch's allocator, except while the
-    current stream is being captured."""
+    grout_attn_prefill_ws with scratch from torch's allocator (up to 17 MB), also
+    while other streams are being captured.  A call that is captured itself, or
+    has no memory left, runs unsplit: the same function with other roundings, so
+    the replay is within the attention tolerance of an eager call, not equal to
+    it.  A graph that is to hold the split records grout_attn_prefill_ws with a
+    workspace of its own."""
     if q.dim() != 3:
         _fail(f"q must be rank 3 [seqlen, heads, head_dim], got {list(q.shape)}")
     q_len, Hq, D = q.shape
